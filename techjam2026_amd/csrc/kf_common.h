@@ -301,8 +301,30 @@ __device__ __forceinline__ int xcd_remap(int bid, int nblocks) {
 // Compute units of the current device (host side, cached; abi.hip).
 int cu_count();
 
+// erf-GELU, x * Phi(x). The lower tail Phi(-a) = erfc(a / sqrt 2) / 2 of a = |x| is one
+// exponential of a polynomial: log2 Phi(-a) is smooth, and a degree-10 minimax fit on [0, 6]
+// (weighted by Phi, so that the error of Phi itself is what is bounded) leaves 3.2e-10 in
+// Phi, far below the rounding of its fp32 evaluation. Past 6 the fit goes on falling (its
+// leading coefficient is negative), so the tail underflows to zero as it should; +-inf and
+// NaN come out as x * Phi(x) gives them. Error against float64 over N(0, 1) inputs, 2-norm:
+// 3.4e-8 relative, 0.5 x (1 + erf(x / sqrt 2)) in fp32 3.7e-8. Twelve VALU instructions and
+// one exponential with no branch, where the library erff takes both of its branches whenever a
+// wavefront's lanes differ (about 40 instructions).
 __device__ __forceinline__ float gelu_erf(float x) {
-  return 0.5f * x * (1.0f + erff(x * 0.70710678118654752440f));
+  const float a = __builtin_fabsf(x);
+  float q = -4.7225789501226245e-08f;
+  q = __builtin_fmaf(q, a, 1.2433845313353231e-06f);
+  q = __builtin_fmaf(q, a, -1.4236356946639717e-05f);
+  q = __builtin_fmaf(q, a, 9.107442747335881e-05f);
+  q = __builtin_fmaf(q, a, -3.168052062392235e-04f);
+  q = __builtin_fmaf(q, a, 5.40691107744351e-05f);
+  q = __builtin_fmaf(q, a, 6.903660949319601e-03f);
+  q = __builtin_fmaf(q, a, -5.242427811026573e-02f);
+  q = __builtin_fmaf(q, a, -4.5922330021858215e-01f);
+  q = __builtin_fmaf(q, a, -1.151104211807251f);
+  q = __builtin_fmaf(q, a, -1.0f);
+  const float e = __builtin_amdgcn_exp2f(q);       // Phi(-|x|)
+  return x * (x < 0.0f ? e : 1.0f - e);
 }
 
 }  // namespace kf
