@@ -170,6 +170,49 @@ int kf_gemm_qkv_tiled(const void* a, const void* a_lo, int a_dtype, int64_t lda,
                       int64_t B, int64_t S, int64_t H, int64_t hd, int mode, int tile,
                       void* stream);
 
+/* kf_layer_block flags */
+enum { KF_LAYER_TAIL = 1, KF_LAYER_QKV = 2 };
+
+/* One 16-bit weight plane [N, K] (row-major, by kf_split) into MFMA fragment order: the
+ * 16-byte piece of row 16 nt + r, columns 32 kt + 8 g .. + 7 goes to piece
+ * (nt * K / 32 + kt) * 64 + 16 g + r, so a wavefront reads its operand of one
+ * v_mfma_f32_16x16x32 as 1 KB of consecutive bytes. N % 16 == 0, K % 32 == 0. No reference
+ * counterpart (a layout of this library's weights, made once). */
+int kf_fragments(const void* src, void* dst, int64_t N, int64_t K, void* stream);
+
+/* Arguments of kf_layer_block. Rows m = b * S + s; [M, d] operands are dense unless a
+ * stride is given; weight planes by kf_split, then kf_fragments; biases fp32; modes are
+ * KF_MMA_F16, KF_MMA_F16X2 or KF_MMA_F16X3. */
+typedef struct {
+  int flags;                                /* KF_LAYER_TAIL | KF_LAYER_QKV (at least one) */
+  int rows;                                 /* rows per block: 16, 32, 64 (32 where there is no
+                                               64-row kernel); 0 = automatic */
+  int64_t M, d, F, S, H, hd;
+  const float* res; int64_t ld_res;         /* residual rows (TAIL), or x */
+  const uint8_t* keep;                      /* [M] row mask, or NULL */
+  const void* ctx_hi; const void* ctx_lo;   /* TAIL: attention output, fp16 plane(s) */
+  const void* wo_hi; const void* wo_lo; const float* bo; int out_mode;
+  const float* norm2_w; const float* norm2_b; float norm2_eps;
+  const void* w1_hi; const void* w1_lo; const float* b1; int f1_mode;
+  const void* w2_hi; const void* w2_lo; const float* b2; int f2_mode;
+  const float* norm_w; const float* norm_b; float norm_eps;
+  float* s_out;                             /* the residual rows after the block, or NULL */
+  const void* wqkv_hi; const void* wqkv_lo; const float* bqkv; int attn_mode;
+  float* q_out; void* k_hi; void* k_lo; void* vt_hi; void* vt_lo; int64_t sp;
+  void* y; int y_dtype;                     /* without QKV: the normalised, masked rows */
+} kf_layer_args;
+
+/* The row-wise part of a narrow layer (d in {32, 64, 96, 128, 192, 256}, F % 32 == 0) in
+ * one launch. With KF_LAYER_TAIL, from the attention output:
+ *   s = (res + ctx . Wo^T + bo) * keep;  h = LN(s; norm2)
+ *   s = (s + gelu(h . W1^T + b1) . W2^T + b2) * keep
+ * (without it s = res * keep); s_out, if given, receives s; h = LN(s; norm). Then with
+ * KF_LAYER_QKV the projections of h in the attention layout of kf_gemm_qkv (k_lo / vt_lo
+ * NULL: one plane each; the pad columns [S, sp) of v^T are zeroed), else y = h * keep in
+ * y_dtype. Replaces kernelforge/optimized.py:483-489 and :560-585 for such widths, where
+ * the reference launches each operation. Row results do not depend on `rows`. */
+int kf_layer_block(const kf_layer_args* args, void* stream);
+
 /* k, v [B, H, S, hd] (strides[4] in elements, unit hd stride; fp32 / fp16 / bf16) into the
  * attention layout of kf_flash_fwd for `mode`: K planes with strides ko_strides (b, h, s, 1)
  * and V^T planes with strides vt_strides (b, h, d, 1), whose columns [S, roundup(S, 8)) it

@@ -21,12 +21,14 @@ OK, EINVAL, EUNSUPPORTED, ELAUNCH, EDEVICE = 0, 1, 2, 3, 4
 LN_HAS_Y, LN_HAS_MASK, LN_MASK_OUT, LN_WRITE_S = 1, 2, 4, 8
 ACT_NONE, ACT_GELU_ERF = 0, 1
 FLASH_CAUSAL, FLASH_SKIP_PAD_ROWS, FLASH_P16, FLASH_ROUND_SCORES, FLASH_NO_PIPE, FLASH_ONE_TILE = 1, 2, 4, 8, 16, 32
+LAYER_TAIL, LAYER_QKV = 1, 2
 ABI_VERSION = 4
 
 EXPORTS = ("kf_abi_version", "kf_last_error", "kf_device_ok", "kf_add_mask_ln", "kf_split",
            "kf_gemm", "kf_gemm_tiled", "kf_gemm_tile_info", "kf_mask_prep", "kf_gemm_qkv",
            "kf_gemm_qkv_tiled", "kf_attn_prep", "kf_flash_tile_info", "kf_flash_block_map",
-           "kf_flash_fwd", "kf_flash_attention_static")
+           "kf_flash_fwd", "kf_flash_attention_static", "kf_layer_block",
+           "kf_fragments")
 
 
 class KernelError(RuntimeError):
@@ -49,6 +51,25 @@ c_int = ctypes.c_int
 c_vp = ctypes.c_void_p
 c_f = ctypes.c_float
 c_i64p = ctypes.POINTER(ctypes.c_int64)
+
+
+class LayerArgs(ctypes.Structure):
+    """kf_layer_args (include/kf950.h), field for field."""
+    _fields_ = [
+        ("flags", c_int), ("rows", c_int),
+        ("M", c_i64), ("d", c_i64), ("F", c_i64), ("S", c_i64), ("H", c_i64), ("hd", c_i64),
+        ("res", c_vp), ("ld_res", c_i64), ("keep", c_vp),
+        ("ctx_hi", c_vp), ("ctx_lo", c_vp),
+        ("wo_hi", c_vp), ("wo_lo", c_vp), ("bo", c_vp), ("out_mode", c_int),
+        ("norm2_w", c_vp), ("norm2_b", c_vp), ("norm2_eps", c_f),
+        ("w1_hi", c_vp), ("w1_lo", c_vp), ("b1", c_vp), ("f1_mode", c_int),
+        ("w2_hi", c_vp), ("w2_lo", c_vp), ("b2", c_vp), ("f2_mode", c_int),
+        ("norm_w", c_vp), ("norm_b", c_vp), ("norm_eps", c_f),
+        ("s_out", c_vp),
+        ("wqkv_hi", c_vp), ("wqkv_lo", c_vp), ("bqkv", c_vp), ("attn_mode", c_int),
+        ("q_out", c_vp), ("k_hi", c_vp), ("k_lo", c_vp), ("vt_hi", c_vp), ("vt_lo", c_vp),
+        ("sp", c_i64), ("y", c_vp), ("y_dtype", c_int),
+    ]
 
 
 def _declare(h: ctypes.CDLL) -> None:
@@ -97,6 +118,10 @@ def _declare(h: ctypes.CDLL) -> None:
     h.kf_flash_attention_static.argtypes = [c_vp, c_i64p, c_vp, c_i64p, c_vp, c_i64p, c_int,
                                             c_vp, c_vp, c_i64p, c_int, c_vp, c_int, c_i64,
                                             c_i64, c_i64, c_i64, c_i64, c_f, c_int, c_int, c_vp]
+    h.kf_fragments.restype = c_int
+    h.kf_fragments.argtypes = [c_vp, c_vp, c_i64, c_i64, c_vp]
+    h.kf_layer_block.restype = c_int
+    h.kf_layer_block.argtypes = [ctypes.POINTER(LayerArgs), c_vp]
 
 
 def available() -> bool:

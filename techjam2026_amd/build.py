@@ -41,6 +41,7 @@ DEVICE_FLAGS = [
 # per element per rescale.
 SOURCE_FLAGS = {
     "flash": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "layer": ["-mllvm", "-amdgpu-mfma-vgpr-form"],    # accumulators feed the row arithmetic
 }
 
 

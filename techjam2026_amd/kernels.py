@@ -361,6 +361,22 @@ class PreparedLinear:
                                   None if self.lo is None else self.lo.data_ptr(), _stream())
             _end(tok)
             L.check("kf_split", st)
+        self._fragments = None
+
+    def fragments(self):
+        """(hi, lo or None) in MFMA fragment order for `layer_block` (kf_fragments), made on
+        the first call and kept with the weight."""
+        if self._fragments is None:
+            planes = []
+            for src in (self.hi, self.lo):
+                dst = None
+                if src is not None:
+                    dst = torch.empty_like(src)
+                    L.check("kf_fragments", L.lib().kf_fragments(src.data_ptr(), dst.data_ptr(),
+                                                                 self.N, self.K, _stream()))
+                planes.append(dst)
+            self._fragments = tuple(planes)
+        return self._fragments
 
 
 def gemm_tiles() -> List[Tuple[int, dict]]:
@@ -451,15 +467,17 @@ class AttnOperands:
 
 
     @staticmethod
-    def empty_stack(B: int, S: int, H: int, Dh: int, mode: int, device) -> "AttnOperands":
-        """Buffers in the layout kf_gemm_qkv writes: q and k token-major [B, S, H, Dh]."""
+    def empty_stack(B: int, S: int, H: int, Dh: int, mode: int, device,
+                    zero_pad: bool = True) -> "AttnOperands":
+        """Buffers in the layout kf_gemm_qkv writes: q and k token-major [B, S, H, Dh].
+        `zero_pad` False: the producer zeroes V^T's pad columns itself (kf_layer_block)."""
         planes = 2 if mode in SPLIT_MODES else 1
         dt = MODE_STORAGE[mode]
         sp = (S + 7) // 8 * 8
         q = torch.empty((B, S, H, Dh), dtype=torch.float32, device=device)
         k = torch.empty((planes, B, S, H, Dh), dtype=dt, device=device)
         vt = torch.empty((planes, B, H, Dh, sp), dtype=dt, device=device)
-        if sp > S:      # kf_flash_fwd reads V^T up to sp: the pad must be finite
+        if zero_pad and sp > S:      # kf_flash_fwd reads V^T up to sp: the pad must be finite
             vt[..., S:].zero_()
         p = lambda t: t.permute(0, 2, 1, 3)  # noqa: E731
         return AttnOperands(p(q), p(k[0]), p(k[planes - 1]) if planes == 2 else None,
@@ -494,6 +512,70 @@ def linear_qkv(h: Act, w: PreparedLinear, B: int, S: int, H: int, Dh: int,
     _end(tok)
     L.check("kf_gemm_qkv", st)
     return ops
+
+
+# ------------------------------------------------------------------ narrow layers
+LAYER_WIDTHS = (32, 64, 96, 128, 192, 256)
+LAYER_MODES = (L.MMA_F16, L.MMA_F16X2, L.MMA_F16X3)
+
+
+def layer_block_supported(d: int, ffn_dim: int, modes) -> bool:
+    """kf_layer_block serves this width, feed-forward width and these stage modes."""
+    return d in LAYER_WIDTHS and ffn_dim % 32 == 0 and all(m in LAYER_MODES for m in modes)
+
+
+def layer_block(res: torch.Tensor, keep: Optional[torch.Tensor], norm, tail=None, qkv=None,
+                want_residual: bool = True, out_dtype: torch.dtype = torch.float32,
+                rows: int = 0):
+    """The row-wise part of a layer in one launch (kf_layer_block).
+
+    `res` [M, d] fp32; `keep` [M] uint8 or None; `norm` (weight, bias, eps) ends the block.
+    `tail` = (ctx, out, norm2, ffn_in, ffn_out): attention output ([M, d] fp16 tensor or
+    Planes, dense), PreparedLinear out_proj, (weight, bias, eps), PreparedLinear x 2.
+    `qkv` = (PreparedLinear, B, S, H, Dh, single): the next projections, as `linear_qkv`.
+    Returns (s or None, AttnOperands) with `qkv`, else (s or None, y [M, d] in `out_dtype`).
+    `rows` forces the rows per block (16 / 32 / 64; 0: automatic; same results)."""
+    M, d = res.shape
+    assert res.dtype == torch.float32 and res.stride(1) == 1
+    _need_cuda(res, keep)
+    dev = res.device
+    s = torch.empty((M, d), dtype=torch.float32, device=dev) if want_residual else None
+    a = L.LayerArgs(flags=0, rows=rows, M=M, d=d, res=res.data_ptr(), ld_res=res.stride(0),
+                    keep=_hi(keep), norm_w=norm[0].data_ptr(), norm_b=norm[1].data_ptr(),
+                    norm_eps=norm[2], s_out=_hi(s))
+    flops, nbytes = 0.0, float(M * d) * (4 + (4 if want_residual else 0))
+    if tail is not None:
+        ctx, out, norm2, f1, f2 = tail
+        a.flags |= L.LAYER_TAIL
+        a.F = f1.N
+        a.ctx_hi, a.ctx_lo = _hi(ctx), _lo(ctx)
+        (a.wo_hi, a.wo_lo), a.bo, a.out_mode = map(_hi, out.fragments()), out.bias.data_ptr(), out.mode
+        a.norm2_w, a.norm2_b, a.norm2_eps = norm2[0].data_ptr(), norm2[1].data_ptr(), norm2[2]
+        (a.w1_hi, a.w1_lo), a.b1, a.f1_mode = map(_hi, f1.fragments()), f1.bias.data_ptr(), f1.mode
+        (a.w2_hi, a.w2_lo), a.b2, a.f2_mode = map(_hi, f2.fragments()), f2.bias.data_ptr(), f2.mode
+        flops += 2.0 * M * (d * d + 2 * d * f1.N)
+        nbytes += M * d * ctx.element_size() + 4 * (d * d + 2 * d * f1.N)
+    if qkv is not None:
+        w, B, S, H, Dh, single = qkv
+        mode = (L.MMA_F16 if single else L.MMA_F16X3 if w.mode == L.MMA_F16X2 else w.mode)
+        ops = AttnOperands.empty_stack(B, S, H, Dh, mode, dev, zero_pad=False)
+        a.flags |= L.LAYER_QKV
+        a.S, a.H, a.hd, a.sp = S, H, Dh, ops.vt_hi.shape[-1]
+        (a.wqkv_hi, a.wqkv_lo), a.bqkv, a.attn_mode = map(_hi, w.fragments()), w.bias.data_ptr(), w.mode
+        a.q_out = ops.q.data_ptr()
+        a.k_hi, a.k_lo, a.vt_hi, a.vt_lo = (_hi(t) for t in (ops.k_hi, ops.k_lo, ops.vt_hi, ops.vt_lo))
+        flops += 6.0 * M * d * d
+        nbytes += M * d * (4 + 4 * (2 if ops.k_lo is not None else 1)) + 12 * d * d
+        result = ops
+    else:
+        result = torch.empty((M, d), dtype=out_dtype, device=dev)
+        a.y, a.y_dtype = result.data_ptr(), _code(result)
+        nbytes += M * d * result.element_size()
+    tok = _begin(f"layer_block[{M}x{d}]", flops, nbytes)
+    st = L.lib().kf_layer_block(ctypes.byref(a), _stream())
+    _end(tok)
+    L.check("kf_layer_block", st)
+    return s, result
 
 
 def k_in_place(k: torch.Tensor, mode: int) -> bool:

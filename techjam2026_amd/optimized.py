@@ -345,6 +345,9 @@ class FusedTransformer(BaselineTransformer):
         res = x.reshape(M, d)
         if io_dtype != torch.float32:        # 16-bit input: widened once, fp32 inside
             res = res.float()
+        if self._rows_fused(rdtype, (m_attn, m_out, m_f1, m_f2)):
+            return self._narrow_stack(res, keep, keep2d, kv_len, prefix, B, S, io_dtype,
+                                      ctx_fmt, single_attn, p16, rs).view(B, S, d)
         res, h = K.add_mask_layernorm(res, None, keep, self.layers[0].norm1.weight,
                                       self.layers[0].norm1.bias, self.layers[0].norm1.eps,
                                       out_dtype=h_attn, residual_dtype=rdtype)
@@ -380,6 +383,50 @@ class FusedTransformer(BaselineTransformer):
                                           out_dtype=io_dtype if last else h_attn,
                                           residual_dtype=rdtype, want_residual=not last)
         return h.view(B, S, d)
+
+    def _rows_fused(self, rdtype, modes) -> bool:
+        """Whether the row-wise part of each layer runs as one kernel (kf_layer_block): a
+        width it serves, fp16-family stages and fp32 norm parameters (16-bit models keep
+        theirs in 16 bits) that it can read in 16-byte pieces."""
+        cfg = self.config
+        norms = [n for layer in self.layers for n in (layer.norm1, layer.norm2)] + [self.final_norm]
+        return (rdtype == torch.float32
+                and K.layer_block_supported(cfg.d_model, cfg.ffn_dim, modes)
+                and all(t.dtype == torch.float32 and t.is_contiguous() and t.data_ptr() % 16 == 0
+                        for n in norms for t in (n.weight, n.bias)))
+
+    def _narrow_stack(self, res, keep, keep2d, kv_len, prefix, B, S, io_dtype, ctx_fmt,
+                      single_attn, p16, rs):
+        """The stack of a narrow model: per layer attention and one row kernel from the
+        attention output to the next layer's q, k, v^T (the last one: to the output)."""
+        cfg = self.config
+        H, Dh = cfg.num_heads, cfg.d_model // cfg.num_heads
+        M = B * S
+
+        def norm(ln):
+            return ln.weight, ln.bias, ln.eps
+
+        def qkv(i):
+            return self._layers_w[i]["qkv"], B, S, H, Dh, single_attn
+
+        if res.stride(1) != 1 or res.stride(0) % 4 or res.data_ptr() % 16:
+            res = res.clone(memory_format=torch.contiguous_format)
+        # the first residual is x itself: the row kernel applies the mask where it reads it
+        _, ops = K.layer_block(res, keep, norm(self.layers[0].norm1), qkv=qkv(0),
+                               want_residual=False)
+        for i, layer in enumerate(self.layers):
+            w = self._layers_w[i]
+            last = i + 1 == len(self.layers)
+            ctx = K._alloc((B, S, H, Dh), ctx_fmt, res.device)
+            K.flash_attention_ops(ops, keep=keep2d, causal=cfg.causal, sm_scale=Dh ** -0.5,
+                                  out=ctx.permute(0, 2, 1, 3), kv_len=kv_len, prefix=prefix,
+                                  skip_pad_rows=keep is not None, p16=p16, round_scores=rs)
+            tail = (ctx.view(M, cfg.d_model), w["out"], norm(layer.norm2), w["ffn_in"], w["ffn_out"])
+            if last:
+                return K.layer_block(res, keep, norm(self.final_norm), tail=tail,
+                                     want_residual=False, out_dtype=io_dtype)[1]
+            res, ops = K.layer_block(res, keep, norm(self.layers[i + 1].norm1), tail=tail,
+                                     qkv=qkv(i + 1))
 
     # --- graph path --------------------------------------------------------------
     def _body(self, x, valid_token_mask):

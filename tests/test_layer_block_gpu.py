@@ -1,0 +1,138 @@
+"""kf_layer_block (the row-wise part of a narrow layer in one launch) against the same
+arithmetic in float64, at the edges of its tiles: rows around a block, hidden widths that are
+not a multiple of the model width, sequences that end inside a store, each width, each stage
+precision; and the independence of its results from the rows per block."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from techjam2026_amd import _lib as L
+from techjam2026_amd import kernels as K
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda")
+
+# Relative error (2-norm) of a product at each precision: fp32 accumulation for f16x3; one
+# fp16 rounding of each operand (2^-11, uniform: / sqrt(3), two operands) for the others.
+TOL = {L.MMA_F16X3: 3e-6, L.MMA_F16X2: 1e-3, L.MMA_F16: 1e-3}
+
+
+def _params(d, F, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+
+    def rnd(*shape):
+        return torch.randn(*shape, device=DEV, generator=g)
+
+    def lin(n, k):
+        return rnd(n, k) * (2.0 / (n + k)) ** 0.5, 0.1 * rnd(n)
+
+    def norm():
+        return (1 + 0.1 * rnd(d)).contiguous(), 0.1 * rnd(d), 1e-5
+
+    return dict(out=lin(d, d), f1=lin(F, d), f2=lin(d, F), qkv=lin(3 * d, d), norm2=norm(),
+                norm=norm()), rnd
+
+
+def _ln(x, n):
+    return torch.nn.functional.layer_norm(x, x.shape[-1:], n[0].double(), n[1].double(), n[2])
+
+
+def _rel(got, want):
+    return float((got.double() - want).norm() / want.norm())
+
+
+def _act(x, mode):
+    """An activation in a stage's operand format."""
+    return K.Planes.from_float(x) if mode == L.MMA_F16X3 else x.half()
+
+
+def _float(a):
+    return a.float() if isinstance(a, torch.Tensor) else a.hi.float() + a.lo.float()
+
+
+def _run(d, F, B, S, H, modes, masked, seed, rows=0):
+    """(outputs of the kernel, float64 results) for tail + QKV, tail + output and QKV alone."""
+    m_attn, m_out, m_f1, m_f2 = modes
+    p, rnd = _params(d, F, seed)
+    M = B * S
+    res, ctx = rnd(M, d), rnd(M, d)
+    keep = (rnd(M) < 0.5).to(torch.uint8) if masked else None
+    w = {n: K.PreparedLinear(*p[n], m) for n, m in
+         (("qkv", m_attn), ("out", m_out), ("f1", m_f1), ("f2", m_f2))}
+    a = _act(ctx, m_out)
+    tail = (a, w["out"], p["norm2"], w["f1"], w["f2"])
+    qkv = (w["qkv"], B, S, H, d // H, False)
+    s, ops = K.layer_block(res, keep, p["norm"], tail=tail, qkv=qkv, rows=rows)
+    _, y = K.layer_block(res, keep, p["norm"], tail=tail, want_residual=False, rows=rows)
+    _, ops0 = K.layer_block(res, keep, p["norm"], qkv=qkv, want_residual=False, rows=rows)
+    kk = 1.0 if keep is None else keep.double()[:, None]
+
+    def lin(x, n):
+        return x @ p[n][0].double().t() + p[n][1].double()
+
+    e = (res.double() + lin(_float(a).double(), "out")) * kk
+    f = lin(_ln(e, p["norm2"]), "f1")
+    f = 0.5 * f * (1 + torch.erf(f * 0.5 ** 0.5))
+    e = (e + lin(f, "f2")) * kk
+    h = _ln(e, p["norm"])
+
+    def split(h):
+        q, k, v = lin(h, "qkv").view(B, S, 3, H, d // H).permute(2, 0, 3, 1, 4)
+        return q, k, v.transpose(-2, -1)
+
+    def got(o):
+        two = o.k_lo is not None
+        return (o.q, o.k_hi.float() + o.k_lo.float() if two else o.k_hi,
+                o.vt_hi.float() + o.vt_lo.float() if two else o.vt_hi)
+
+    return ((s, y, *got(ops), *got(ops0)),
+            (e, h * kk, *split(h), *split(_ln(res.double() * kk, p["norm"]))), S)
+
+
+def _check(outs, tol, what):
+    got, want, S = outs
+    for i, (g, w) in enumerate(zip(got, want)):
+        if g.dim() == 4 and g.shape[-1] != w.shape[-1]:            # v^T: zeroed pad columns
+            assert torch.count_nonzero(g[..., S:]) == 0, f"{what}: pad columns of output {i}"
+            g = g[..., :S]
+        assert _rel(g, w) < tol, f"{what}: output {i} off by {_rel(g, w):.2e}"
+
+
+X3 = (L.MMA_F16X3,) * 4
+CASES = [
+    (32, 32, 1, 1, 4, X3, False), (32, 96, 3, 37, 1, X3, True), (64, 256, 2, 65, 8, X3, True),
+    (64, 32, 1, 200, 2, X3, False), (96, 160, 2, 63, 3, X3, True), (128, 128, 1, 16, 4, X3, False),
+    (128, 512, 3, 129, 1, X3, True), (128, 64, 2, 100, 16, X3, True), (192, 768, 5, 33, 6, X3, True),
+    (192, 192, 1, 31, 24, X3, False), (256, 1024, 2, 130, 4, X3, True), (256, 32, 1, 17, 1, X3, False),
+    (128, 160, 2, 60, 2, (L.MMA_F16X3, L.MMA_F16, L.MMA_F16, L.MMA_F16), True),
+    (64, 256, 2, 66, 8, (L.MMA_F16X3, L.MMA_F16X2, L.MMA_F16X3, L.MMA_F16X2), True),
+    (256, 1024, 1, 77, 4, (L.MMA_F16, L.MMA_F16X3, L.MMA_F16X2, L.MMA_F16X3), False),
+    (32, 64, 2, 9, 4, (L.MMA_F16X2, L.MMA_F16, L.MMA_F16X3, L.MMA_F16), True),
+    (96, 96, 1, 70, 6, (L.MMA_F16,) * 4, False),
+]
+
+
+@pytest.mark.parametrize("d,F,B,S,H,modes,masked", CASES)
+def test_row_block_matches_float64(d, F, B, S, H, modes, masked):
+    for rows in (0, 16, 32, 64):
+        print(f"d{d} F{F} B{B} S{S} H{H} {modes} rows {rows}", flush=True)
+        outs = _run(d, F, B, S, H, modes, masked, 1, rows)
+        # every output passes each stage once or more: the roundings of the stages add
+        tol = 2 * max(TOL[m] for m in modes)
+        _check(outs, tol, f"rows {rows}")
+        if rows == 0:
+            first = outs[0]
+        else:
+            for i, (a, b) in enumerate(zip(first, outs[0])):
+                assert torch.equal(a, b), f"output {i} differs between rows 0 and {rows}"
+
+
+def test_single_plane_operands_are_the_rounded_values():
+    """An f16x3 projection for single-pass attention writes the hi planes alone."""
+    p, rnd = _params(64, 64, 3)
+    x = rnd(2 * 50, 64)
+    w = K.PreparedLinear(*p["qkv"], L.MMA_F16X3)
+    two = K.layer_block(x, None, p["norm"], qkv=(w, 2, 50, 2, 32, False))[1]
+    one = K.layer_block(x, None, p["norm"], qkv=(w, 2, 50, 2, 32, True))[1]
+    assert one.k_lo is None and torch.equal(one.k_hi, two.k_hi) and torch.equal(one.vt_hi, two.vt_hi)
