@@ -142,7 +142,13 @@ def _alloc(shape, fmt, device) -> Act:
     return torch.empty(shape, dtype=fmt, device=device)
 
 
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream() -> int:
+    """The current stream's handle (without building a torch.cuda.Stream: 0.4 against 2.8 us)."""
+    if _raw_stream is not None:
+        return _raw_stream(torch.cuda.current_device())
     return torch.cuda.current_stream().cuda_stream
 
 
@@ -279,12 +285,15 @@ def add_mask_layernorm(x: torch.Tensor, y: Optional[torch.Tensor],
                        out_dtype=None,
                        residual_dtype: Optional[torch.dtype] = None,
                        want_residual: bool = True,
+                       s_out: Optional[torch.Tensor] = None, h_out: Optional[Act] = None,
                        ) -> Tuple[Optional[torch.Tensor], Act]:
     """(s, h) with s = (x + y) * keep and h = LayerNorm(s) [* keep when mask_out].
 
     Signature and semantics of `kernelforge/ops/layernorm.py:101-156`. x, y: [M, d]
     (unit column stride); keep: [M] 0/1 (bool, uint8 or float) or None. `out_dtype` may
     be a torch dtype or a PlanesFormat (F16X2 / BF16X2), which returns h as Planes.
+    `s_out` / `h_out`: write s and h into these ([M, d], of those dtypes, unit column
+    stride) instead of new tensors.
     """
     assert x.dim() == 2, "pass [M, d]"
     _need_cuda(x, y, keep, weight, bias)
@@ -304,8 +313,12 @@ def add_mask_layernorm(x: torch.Tensor, y: Optional[torch.Tensor],
         if keep.dtype == torch.bool:
             keep = keep.view(torch.uint8)
         keep = keep.contiguous()
-    s = torch.empty((M, d), dtype=residual_dtype, device=x.device) if want_residual else None
-    h = _alloc((M, d), out_dtype, x.device)
+    s = None
+    if want_residual:
+        s = s_out if s_out is not None else torch.empty((M, d), dtype=residual_dtype, device=x.device)
+        assert tuple(s.shape) == (M, d) and s.dtype == residual_dtype and s.stride(1) == 1
+    h = h_out if h_out is not None else _alloc((M, d), out_dtype, x.device)
+    assert tuple(h.shape) == (M, d) and h.stride(1) == 1
     flags = ((L.LN_HAS_Y if y is not None else 0) | (L.LN_HAS_MASK if keep is not None else 0)
              | (L.LN_MASK_OUT if mask_out else 0) | (L.LN_WRITE_S if want_residual else 0))
     nbytes = M * d * (x.element_size() + (y.element_size() if y is not None else 0)
@@ -524,58 +537,76 @@ def layer_block_supported(d: int, ffn_dim: int, modes) -> bool:
     return d in LAYER_WIDTHS and ffn_dim % 32 == 0 and all(m in LAYER_MODES for m in modes)
 
 
-def layer_block(res: torch.Tensor, keep: Optional[torch.Tensor], norm, tail=None, qkv=None,
-                want_residual: bool = True, out_dtype: torch.dtype = torch.float32,
-                rows: int = 0):
-    """The row-wise part of a layer in one launch (kf_layer_block).
+class LayerBlock:
+    """The row-wise part of a layer as one launch (kf_layer_block), prepared: everything but
+    the residual rows and the output is fixed, so a call sets two pointers and launches.
 
-    `res` [M, d] fp32; `keep` [M] uint8 or None; `norm` (weight, bias, eps) ends the block.
+    M rows of width d; `keep` [M] uint8 or None; `norm` (weight, bias, eps) ends the block.
     `tail` = (ctx, out, norm2, ffn_in, ffn_out): attention output ([M, d] fp16 tensor or
     Planes, dense), PreparedLinear out_proj, (weight, bias, eps), PreparedLinear x 2.
     `qkv` = (PreparedLinear, B, S, H, Dh, single): the next projections, as `linear_qkv`.
-    Returns (s or None, AttnOperands) with `qkv`, else (s or None, y [M, d] in `out_dtype`).
+    A call takes res [M, d] (fp32, unit column stride, 16-byte aligned rows) and returns
+    (s or None, AttnOperands) with `qkv`, else (s or None, y [M, d] in `out_dtype`); s and the
+    operands are buffers of this object, written again by each call, y is a new tensor.
     `rows` forces the rows per block (16 / 32 / 64; 0: automatic; same results)."""
-    M, d = res.shape
-    assert res.dtype == torch.float32 and res.stride(1) == 1
-    _need_cuda(res, keep)
-    dev = res.device
-    s = torch.empty((M, d), dtype=torch.float32, device=dev) if want_residual else None
-    a = L.LayerArgs(flags=0, rows=rows, M=M, d=d, res=res.data_ptr(), ld_res=res.stride(0),
-                    keep=_hi(keep), norm_w=norm[0].data_ptr(), norm_b=norm[1].data_ptr(),
-                    norm_eps=norm[2], s_out=_hi(s))
-    flops, nbytes = 0.0, float(M * d) * (4 + (4 if want_residual else 0))
-    if tail is not None:
-        ctx, out, norm2, f1, f2 = tail
-        a.flags |= L.LAYER_TAIL
-        a.F = f1.N
-        a.ctx_hi, a.ctx_lo = _hi(ctx), _lo(ctx)
-        (a.wo_hi, a.wo_lo), a.bo, a.out_mode = map(_hi, out.fragments()), out.bias.data_ptr(), out.mode
-        a.norm2_w, a.norm2_b, a.norm2_eps = norm2[0].data_ptr(), norm2[1].data_ptr(), norm2[2]
-        (a.w1_hi, a.w1_lo), a.b1, a.f1_mode = map(_hi, f1.fragments()), f1.bias.data_ptr(), f1.mode
-        (a.w2_hi, a.w2_lo), a.b2, a.f2_mode = map(_hi, f2.fragments()), f2.bias.data_ptr(), f2.mode
-        flops += 2.0 * M * (d * d + 2 * d * f1.N)
-        nbytes += M * d * ctx.element_size() + 4 * (d * d + 2 * d * f1.N)
-    if qkv is not None:
-        w, B, S, H, Dh, single = qkv
-        mode = (L.MMA_F16 if single else L.MMA_F16X3 if w.mode == L.MMA_F16X2 else w.mode)
-        ops = AttnOperands.empty_stack(B, S, H, Dh, mode, dev, zero_pad=False)
-        a.flags |= L.LAYER_QKV
-        a.S, a.H, a.hd, a.sp = S, H, Dh, ops.vt_hi.shape[-1]
-        (a.wqkv_hi, a.wqkv_lo), a.bqkv, a.attn_mode = map(_hi, w.fragments()), w.bias.data_ptr(), w.mode
-        a.q_out = ops.q.data_ptr()
-        a.k_hi, a.k_lo, a.vt_hi, a.vt_lo = (_hi(t) for t in (ops.k_hi, ops.k_lo, ops.vt_hi, ops.vt_lo))
-        flops += 6.0 * M * d * d
-        nbytes += M * d * (4 + 4 * (2 if ops.k_lo is not None else 1)) + 12 * d * d
-        result = ops
-    else:
-        result = torch.empty((M, d), dtype=out_dtype, device=dev)
-        a.y, a.y_dtype = result.data_ptr(), _code(result)
-        nbytes += M * d * result.element_size()
-    tok = _begin(f"layer_block[{M}x{d}]", flops, nbytes)
-    st = L.lib().kf_layer_block(ctypes.byref(a), _stream())
-    _end(tok)
-    L.check("kf_layer_block", st)
-    return s, result
+
+    def __init__(self, M: int, d: int, device, keep: Optional[torch.Tensor], norm, tail=None,
+                 qkv=None, want_residual: bool = True, out_dtype: torch.dtype = torch.float32,
+                 rows: int = 0):
+        _need_cuda(keep)
+        self.s = torch.empty((M, d), dtype=torch.float32, device=device) if want_residual else None
+        self.ops = None
+        self.out_dtype = out_dtype
+        self.holds = (keep, norm, tail, qkv)     # the tensors behind the pointers
+        a = self.args = L.LayerArgs(flags=0, rows=rows, M=M, d=d, keep=_hi(keep),
+                                    norm_w=norm[0].data_ptr(), norm_b=norm[1].data_ptr(),
+                                    norm_eps=norm[2], s_out=_hi(self.s))
+        flops, nbytes = 0.0, float(M * d) * (4 + (4 if want_residual else 0))
+        if tail is not None:
+            ctx, out, norm2, f1, f2 = tail
+            a.flags |= L.LAYER_TAIL
+            a.F = f1.N
+            a.ctx_hi, a.ctx_lo = _hi(ctx), _lo(ctx)
+            (a.wo_hi, a.wo_lo), a.bo, a.out_mode = map(_hi, out.fragments()), out.bias.data_ptr(), out.mode
+            a.norm2_w, a.norm2_b, a.norm2_eps = norm2[0].data_ptr(), norm2[1].data_ptr(), norm2[2]
+            (a.w1_hi, a.w1_lo), a.b1, a.f1_mode = map(_hi, f1.fragments()), f1.bias.data_ptr(), f1.mode
+            (a.w2_hi, a.w2_lo), a.b2, a.f2_mode = map(_hi, f2.fragments()), f2.bias.data_ptr(), f2.mode
+            flops += 2.0 * M * (d * d + 2 * d * f1.N)
+            nbytes += M * d * ctx.element_size() + 4 * (d * d + 2 * d * f1.N)
+        if qkv is not None:
+            w, B, S, H, Dh, single = qkv
+            mode = (L.MMA_F16 if single else L.MMA_F16X3 if w.mode == L.MMA_F16X2 else w.mode)
+            ops = self.ops = AttnOperands.empty_stack(B, S, H, Dh, mode, device, zero_pad=False)
+            a.flags |= L.LAYER_QKV
+            a.S, a.H, a.hd, a.sp = S, H, Dh, ops.vt_hi.shape[-1]
+            (a.wqkv_hi, a.wqkv_lo), a.bqkv, a.attn_mode = map(_hi, w.fragments()), w.bias.data_ptr(), w.mode
+            a.q_out = ops.q.data_ptr()
+            a.k_hi, a.k_lo, a.vt_hi, a.vt_lo = (_hi(t) for t in (ops.k_hi, ops.k_lo, ops.vt_hi, ops.vt_lo))
+            flops += 6.0 * M * d * d
+            nbytes += M * d * (4 + 4 * (2 if ops.k_lo is not None else 1)) + 12 * d * d
+        else:
+            nbytes += M * d * out_dtype.itemsize
+        self.work = (f"layer_block[{M}x{d}]", flops, nbytes)
+
+    def __call__(self, res: torch.Tensor):
+        a = self.args
+        assert res.is_cuda and res.dtype == torch.float32 and tuple(res.shape) == (a.M, a.d) \
+            and res.stride(1) == 1
+        a.res, a.ld_res = res.data_ptr(), res.stride(0)
+        result = self.ops
+        if result is None:
+            result = torch.empty((a.M, a.d), dtype=self.out_dtype, device=res.device)
+            a.y, a.y_dtype = result.data_ptr(), _DT[self.out_dtype]
+        tok = _begin(*self.work)
+        st = L.lib().kf_layer_block(ctypes.byref(a), _stream())
+        _end(tok)
+        L.check("kf_layer_block", st)
+        return self.s, result
+
+
+def layer_block(res: torch.Tensor, keep: Optional[torch.Tensor], norm, **options):
+    """One call of a `LayerBlock` for these rows: (s or None, AttnOperands or y)."""
+    return LayerBlock(*res.shape, res.device, keep, norm, **options)(res)
 
 
 def k_in_place(k: torch.Tensor, mode: int) -> bool:
