@@ -16,46 +16,72 @@ __global__ void split_kernel(const float* src, int64_t n, E* hi, E* lo) {
   }
 }
 
-// Automatic choice for 16-bit operands, from per-call sweeps of the layer's GEMM shapes
-// on MI355X at the precisions the plans use (C2, C4, C5). Short K (head-sized) takes small
-// tiles (128 x 64 for the QKV epilogue), N <= 64 the 128 x 64 x 64 tile. Where K is a
-// multiple of 64 a stage carries 64 k (two 32-k sub-tiles, both halves of each 128-byte
-// line copied back to back): 128 x 128 x 64 in two stages is the best or within 4 % of
-// it everywhere (C2 QKV 56.7 -> 49.8 us, ffn_in 45.4 -> 35.0, C4 out_proj 110.7 -> 92.5,
-// C5 ffn_in 1080 -> 976) except on large grids where the weight has more planes than the
-// activation (f16x2: 256 x 128, C4 QKV 542 -> 473), carries split planes on both sides
-// (f16x3: 128 x 256 x 32; for both, 256 x 256 x 32 in two stages with single-buffered
-// fragments where N >= 512: C5 QKV 4477 -> 4069 us, ffn_out 1580 -> 1427, C4 QKV 596 -> 536,
-// out_proj 231 -> 194, an f16x3 ffn_in with GELU 887 -> 790, C5 out_proj (f16x2) 1067 ->
-// 1004; one-round grids such as C2's run it 1.5-2.6x slower), or K is long (fp16,
-// K >= 4096: 256 x 256 x 64 in two stages, 64 x 128 per wavefront, C4 ffn_out 331 -> 320
-// with 128 x 256 x 64 in three stages, then 324 -> 258 with 256 x 256).
-static int pick_dma(int64_t M, int64_t N, int64_t K, int mode, bool qkv) {
-  const int64_t t128 = ((M + 127) / 128) * ((N + 127) / 128);
-  const bool split = mode == KF_MMA_F16X3 || mode == KF_MMA_BF16X3;
-  if (K < 128) return qkv ? DMA_128x64k32s3w4 : DMA_64x64k32s3w4;
-  if (N <= 64 && K % 64 == 0) return DMA_128x64k64s3w8;
-  if (K % 64 == 0) {
-    if (t128 >= 1024) {
-      if (mode == KF_MMA_F16X2) return N >= 512 ? DMA_256x256k32s2w8 : DMA_256x128k64s2w8;
-      if (split) return N >= 512 ? DMA_256x256k32s2w8 : DMA_128x256k32s3w8;
-      if (K >= 4096) return qkv ? DMA_128x256k64s3w8 : DMA_256x256k64s2w8;
-    }
-    return DMA_128x128k64s2w8;
+// Automatic choice for 16-bit operands. Short K (head-sized) takes small tiles (128 x 64 for
+// the QKV epilogue). Otherwise the tile with the least modelled time
+//   q (a K + e s),   q = ceil(tiles / CUs),
+// where a block of the tile spends a us per 1024 of K and e us in its epilogue, and s is the
+// epilogue's weight (plain, GELU, QKV). q is what a whole-chip rule cannot see: tiles of
+// 128 x 128 for 3001 x 768 outputs leave 112 of 256 CUs idle, 256 x 256 ones for 8192 x 3072
+// run a second round half empty. Two blocks sharing a CU take about twice as long as one, so
+// residency does not enter. a, e and s are fitted per operand planes to every tile timed over 60
+// to 64 products (M 64 ... 70000, N and K 256 ... 4096, three epilogues); over those products
+// the choice is within 1-2 % of the fastest tile (geometric mean), 20-25 % faster than a
+// fixed preference for 128 x 128 and, on large grids, 256 x 256 tiles, and never more than
+// 11 % slower than it. Measured, before -> after: f16x3 256 x 512 x 2048 35.8 -> 9.8 us,
+// 1024 x 768 x 3072 59 -> 24; fp16 3001 x 768 x 3072 34.7 -> 30.7, 8192 x 4096 x 1024
+// 101 -> 75; f16x2 8192 x 768 x 3072 92 -> 72.
+struct TileCost { int tile; float a, e; };
+struct ModeCost { float s[3]; TileCost tiles[11]; int n; };
+static const ModeCost kCostSplit = {{1.0f, 1.8f, 1.5f},
+    {{DMA_256x256k32s2w8, 65.f, 7.9f}, {DMA_128x256k32s3w8, 37.f, 4.4f},
+     {DMA_128x128k64s2w8, 20.f, 1.9f}, {DMA_128x64k64s3w8, 13.f, 1.0f},
+     {DMA_64x64k64s4w4, 9.2f, 0.85f}, {DMA_32x64k128s3w4, 6.0f, 0.62f},
+     {DMA_32x32k128s3w4, 3.9f, 0.29f}, {DMA_128x128k32s3w8, 22.f, 2.1f},
+     {DMA_64x64k32s3w4, 10.f, 0.3f}}, 9};
+static const ModeCost kCostSingle = {{1.0f, 1.4f, 1.2f},
+    {{DMA_256x256k64s2w8, 22.f, 9.5f}, {DMA_128x256k64s3w8, 13.f, 4.7f},
+     {DMA_128x128k64s2w8, 8.4f, 1.3f}, {DMA_128x64k64s3w8, 5.4f, 0.72f},
+     {DMA_64x64k64s4w4, 3.5f, 0.34f}, {DMA_32x64k128s3w4, 2.4f, 0.28f},
+     {DMA_32x32k128s3w4, 1.6f, 0.1f}, {DMA_128x256k32s3w8, 15.f, 5.2f},
+     {DMA_128x128k32s3w8, 9.6f, 1.6f}, {DMA_64x64k32s3w4, 5.3f, 0.3f},
+     {DMA_128x128k64s4w8, 8.0f, 2.0f}}, 11};
+static const ModeCost kCostF16x2 = {{1.0f, 1.4f, 1.6f},
+    {{DMA_256x256k32s2w8, 43.f, 7.8f}, {DMA_256x128k64s2w8, 22.f, 4.2f},
+     {DMA_128x128k64s2w8, 15.f, 1.6f}, {DMA_128x64k64s3w8, 8.5f, 1.1f},
+     {DMA_64x64k64s4w4, 6.6f, 0.9f}, {DMA_32x64k128s3w4, 4.5f, 0.6f},
+     {DMA_32x32k128s3w4, 2.6f, 0.3f}, {DMA_256x128k32s3w8, 24.f, 4.5f},
+     {DMA_128x128k32s3w8, 15.f, 2.1f}, {DMA_64x64k32s3w4, 8.5f, 0.3f}}, 10};
+enum { EPI_PLAIN = 0, EPI_GELU = 1, EPI_QKV = 2 };
+
+static int pick_dma(int64_t M, int64_t N, int64_t K, int mode, int epilogue) {
+  if (K < 128) return epilogue == EPI_QKV ? DMA_128x64k32s3w4 : DMA_64x64k32s3w4;
+  const ModeCost& mc = mode == KF_MMA_F16X3 || mode == KF_MMA_BF16X3 ? kCostSplit
+                     : mode == KF_MMA_F16X2 ? kCostF16x2 : kCostSingle;
+  const int64_t cus = cu_count();
+  int best = DMA_128x128k32s4w8;
+  float least = 3.4e38f;
+  for (int i = 0; i < mc.n; ++i) {
+    const TileInfo& t = kTileInfo[mc.tiles[i].tile];
+    if (K % t.bk) continue;
+    const int64_t tiles = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+    // four stages hide the memory latency of a lone block over a long K (fp16 3001 x 768 x
+    // 3072: 34.9 -> 29.7 us), but they leave no room for a second one
+    if (mc.tiles[i].tile == DMA_128x128k64s4w8 && tiles > cus) continue;
+    const float cost = (float)((tiles + cus - 1) / cus) *
+                       (mc.tiles[i].a * (float)K * (1.0f / 1024.0f) + mc.tiles[i].e * mc.s[epilogue]);
+    if (cost < least) { least = cost; best = mc.tiles[i].tile; }
   }
-  if (t128 >= 1024) return mode == KF_MMA_F16X2 ? DMA_256x128k32s3w8 : DMA_128x256k32s3w8;
-  if (N <= 512) return DMA_128x128k32s3w8;
-  return DMA_128x128k32s4w8;
+  return best;
 }
 
 // The tile a call runs: the caller's explicit choice where it applies to the operands
 // (an LDS-DMA tile needs 16-bit A and K a multiple of its BK; f16x2 runs on LDS-DMA tiles
 // only), else the automatic one.
-static int pick_tile(int requested, int64_t M, int64_t N, int64_t K, bool a16, int mode, bool qkv) {
+static int pick_tile(int requested, int64_t M, int64_t N, int64_t K, bool a16, int mode, int epilogue) {
   int t = requested;
   if (t >= DMA_FIRST && (!a16 || K % kTileInfo[t].bk)) t = TILE_AUTO;
   if (mode == KF_MMA_F16X2 && t != TILE_AUTO && t < DMA_FIRST) t = TILE_AUTO;
-  if (t == TILE_AUTO && a16 && K % 32 == 0) t = pick_dma(M, N, K, mode, qkv);
+  if (t == TILE_AUTO && a16 && K % 32 == 0) t = pick_dma(M, N, K, mode, epilogue);
   if (t == TILE_AUTO) {
     const int64_t blocks128 = ((M + 127) / 128) * ((N + 127) / 128);
     if (blocks128 >= 512) t = TILE_128x128k32;
@@ -154,7 +180,8 @@ extern "C" int kf_gemm_tiled(const void* a, const void* a_lo, int a_dtype, int64
              (int)M, (int)N, (int)K, act,
              nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0, wide16};
   hipStream_t st = (hipStream_t)stream;
-  const int t = pick_tile(tile, M, N, K, a_dtype != KF_F32, mode, false);
+  const int t = pick_tile(tile, M, N, K, a_dtype != KF_F32, mode,
+                          act == KF_ACT_GELU_ERF ? EPI_GELU : EPI_PLAIN);
   if (mode == KF_MMA_F16X2 && !is_dma_tile(t)) {
     kf_set_error("kf_gemm: f16x2 needs the LDS-DMA path (fp16 A, K %% 32 == 0; K=%lld)",
                  (long long)K);
@@ -247,7 +274,7 @@ extern "C" int kf_gemm_qkv_tiled(const void* a, const void* a_lo, int a_dtype, i
              q_out, k_hi, k_lo, vt_hi, vt_lo, kv_dtype, sp, (int)S, (int)H, (int)hd, wide16,
              log2_or_neg(S), log2_or_neg(hd)};
   hipStream_t st = (hipStream_t)stream;
-  const int t = pick_tile(tile, M, 3 * d, d, a_dtype != KF_F32, mode, true);
+  const int t = pick_tile(tile, M, 3 * d, d, a_dtype != KF_F32, mode, EPI_QKV);
   if (mode == KF_MMA_F16X2 && !is_dma_tile(t)) {
     kf_set_error("kf_gemm_qkv: f16x2 needs the LDS-DMA path (fp16 A, d %% 32 == 0; d=%lld)",
                  (long long)d);

@@ -1012,7 +1012,9 @@ enum {
   DMA_128x128k32s3w8 = 12, DMA_128x64k64s3w8 = 13, DMA_128x128k64s2w4 = 14,
   DMA_128x128k64s2w8 = 15, DMA_128x256k64s2w8 = 16, DMA_128x256k64s3w8 = 17,
   DMA_256x128k64s2w8 = 18, DMA_256x256k64s2w8 = 19, DMA_256x256k32s2w8 = 20,
-  TILE_LAST = 20
+  DMA_64x64k64s4w4 = 21, DMA_32x64k128s3w4 = 22, DMA_32x32k128s3w4 = 23,
+  DMA_128x128k64s4w8 = 24,
+  TILE_LAST = 24
 };
 
 // (BM, BN, BK, stages, wavefronts, LDS-DMA) of every tile id, in id order; the launch
@@ -1027,6 +1029,8 @@ constexpr TileInfo kTileInfo[TILE_LAST + 1] = {
     {128, 128, 32, 3, 8, 1}, {128, 64, 64, 3, 8, 1}, {128, 128, 64, 2, 4, 1},
     {128, 128, 64, 2, 8, 1}, {128, 256, 64, 2, 8, 1}, {128, 256, 64, 3, 8, 1},
     {256, 128, 64, 2, 8, 1}, {256, 256, 64, 2, 8, 1}, {256, 256, 32, 2, 8, 1},
+    {64, 64, 64, 4, 4, 1}, {32, 64, 128, 3, 4, 1}, {32, 32, 128, 3, 4, 1},
+    {128, 128, 64, 4, 8, 1},
 };
 
 template <int MODE, int AT, class C, int EPI>
@@ -1083,6 +1087,10 @@ static void launch_tile(const GemmArgs& g, int tile, hipStream_t st) {
       case DMA_256x128k64s2w8: return launch_dma<MODE, DmaCfg<256, 128, 64, 2, 4, 2>, EPI>(g, st);
       case DMA_256x256k64s2w8: return launch_dma<MODE, DmaCfg<256, 256, 64, 2, 4, 2>, EPI>(g, st);
       case DMA_256x256k32s2w8: return launch_dma<MODE, DmaCfg<256, 256, 32, 2, 4, 2>, EPI>(g, st);
+      case DMA_64x64k64s4w4: return launch_dma<MODE, DmaCfg<64, 64, 64, 4, 2, 2>, EPI>(g, st);
+      case DMA_32x64k128s3w4: return launch_dma<MODE, DmaCfg<32, 64, 128, 3, 2, 2>, EPI>(g, st);
+      case DMA_128x128k64s4w8: return launch_dma<MODE, DmaCfg<128, 128, 64, 4, 2, 4>, EPI>(g, st);
+      case DMA_32x32k128s3w4: return launch_dma<MODE, DmaCfg<32, 32, 128, 3, 2, 2>, EPI>(g, st);
       default: break;
     }
   }
