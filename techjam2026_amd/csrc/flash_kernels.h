@@ -55,21 +55,19 @@ struct FlashArgs {
   float scale_log2;
   float scale;           // sm_scale itself (score-rounding variant)
   int flags;
+  int only_general;      // flash_general_kernel: prefix-mask rows are another kernel's
 };
 
 constexpr float kNegInf = -__builtin_huge_valf();
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLazy = 8.0f;     // log2 units: probabilities stay <= 256
 
-// GMT: the general-mask instantiation's tile (same block height, so one grid serves both)
-template <int HDP, int P = 2, bool GMT = false> struct FlashTile {
-  // hd 64 in the split modes, prefix masks: eight wavefronts of one 16-row group (the same
+template <int HDP, int P = 2> struct FlashTile {
+  // hd 64 in the split modes: eight wavefronts of one 16-row group (the same
   // 128-row block as four of two groups) at ~100-126 VGPRs, so two blocks give each SIMD
   // four wavefronts instead of two (C2-shape f16x3 attention 28.0 -> 25.3 us, outputs
-  // bit-identical: each row takes the same MFMAs and softmax steps in the same order). The
-  // general-mask launch, empty on prefix masks, keeps 256-thread blocks: with 512 its empty
-  // launch over C5's 32768 blocks took 75.5 instead of 44.7 us.
-  static constexpr bool kWide64 = HDP == 64 && P == 2 && !GMT;
+  // bit-identical: each row takes the same MFMAs and softmax steps in the same order).
+  static constexpr bool kWide64 = HDP == 64 && P == 2;
   static constexpr int BN = HDP >= 256 ? 32 : 64;   // keys per LDS stage
   static constexpr int QG = HDP >= 256 || kWide64 ? 1 : 2;   // 16-row query groups per wavefront
   // Measured on MI355X (B4 H16 S8192 causal): hd >= 128 gains from eight wavefronts
@@ -84,21 +82,6 @@ template <int HDP, int P = 2, bool GMT = false> struct FlashTile {
   static constexpr int STAGES = (HDP >= 256 && P == 1) ? 4 : (HDP >= 128 && 3 * STAGE_BYTES <= 160 * 1024) ? 3 : 2;
   static_assert(BM == (HDP >= 256 ? 128 : HDP >= 128 ? 256 : 128), "one block height per head dim");
 };
-
-// keep[row + key0 + e] for e < 8 (keys past S clamped to S - 1), one dtype dispatch.
-template <typename T>
-__device__ __forceinline__ void keep8_t(const T* p, int key0, int S, float* out) {
-#pragma unroll
-  for (int e = 0; e < 8; ++e) out[e] = (float)p[min(key0 + e, S - 1)];
-}
-__device__ __forceinline__ void load_keep8(const FlashArgs& a, int64_t row, int key0, float* out) {
-  switch (a.keep_dtype) {
-    case KF_U8: keep8_t((const uint8_t*)a.keep + row, key0, a.S, out); break;
-    case KF_F32: keep8_t((const float*)a.keep + row, key0, a.S, out); break;
-    case KF_F16: keep8_t((const _Float16*)a.keep + row, key0, a.S, out); break;
-    default: keep8_t((const __bf16*)a.keep + row, key0, a.S, out); break;
-  }
-}
 
 __device__ __forceinline__ void store_o4(const FlashArgs& a, int64_t off, const float* v) {
   store4_any(a.o, a.o_lo, a.o_dtype, off, v);
@@ -177,14 +160,16 @@ template <int HDP> __host__ __device__ constexpr int vswz(int row) {
   else return b5 | (b3 << 1) | (b1 << 2);
 }
 
-// GM: general key masks (keep read per key) or prefix masks (validity from kv_len alone).
 // VAR: kVarP16 -- split modes carry P as one rounded plane instead of hi + lo
 // (KF_FLASH_P16); kVarRoundScores -- q.k is rounded to the mode's 16-bit type, scaled,
 // and rounded again before the softmax, as the reference's narrow forward computes
 // `matmul(q, k^T) * scale` (KF_FLASH_ROUND_SCORES).
-// The host launches the prefix instantiation and, when a keep mask is given, the general
-// one; each block serves only the batch rows of its kind, so the common path carries no
-// per-key mask loads.
+// Key masks: where a batch row's valid keys are a prefix (kv_len / prefix of kf_mask_prep),
+// validity is a compare with kv_len; else ("general") a tile's keep values are read one
+// per lane, a tile ahead, and balloted into a wave-uniform bit mask that the tile's masked
+// path tests. One kernel serves both kinds of row: a second launch for the general rows,
+// empty on the usual masks, took 3-5 us a layer on small grids and 57 us over 40000 blocks,
+// and its per-key loads made a general row of 333 keys 23 us where the prefix path takes 12.
 constexpr int kVarNone = 0, kVarP16 = 1, kVarRoundScores = 2;
 
 template <typename E> __device__ __forceinline__ float round_to(float v) { return (float)(E)v; }
@@ -243,24 +228,23 @@ __host__ __device__ inline FlashBlock flash_block_map(int bid, int nblocks, int 
   return m;
 }
 
-template <int MODE, int QT, int HDP, bool GM, int VAR = kVarNone>
-__global__ __launch_bounds__((FlashTile<HDP, ModeTraits<MODE>::split ? 2 : 1, GM>::NTH))
-void flash_fwd_kernel(FlashArgs a) {
+// GEN: whether this instantiation serves general rows.
+template <int MODE, int QT, int HDP, int VAR, bool GEN>
+__device__ __forceinline__ void flash_fwd_block(const FlashArgs& a, int bid, int nblocks,
+                                                typename ModeTraits<MODE>::elem* smem) {
   using TR = ModeTraits<MODE>;
   static_assert(VAR != kVarP16 || MODE == MODE_F16X3, "single-plane P is an f16x3 option");
   static_assert(VAR != kVarRoundScores || MODE == MODE_F16 || MODE == MODE_BF16,
                 "score rounding follows a single-pass 16-bit mode");
   constexpr bool PS = VAR != kVarP16;         // P as hi + lo in split modes
   // two query groups pipelined within a tile (their K and V^T fragments held in registers
-  // for both): where those fit beside the rest -- head_dim <= 64 with prefix masks (the
-  // general-mask variant would fall to one wavefront per SIMD)
-  constexpr bool kPipe = FlashTile<HDP, TR::split ? 2 : 1, GM>::QG == 2 && HDP <= 64 && !GM;
+  // for both): where those fit beside the rest (head_dim <= 64)
+  constexpr bool kPipe = FlashTile<HDP, TR::split ? 2 : 1>::QG == 2 && HDP <= 64;
   constexpr bool RS = VAR == kVarRoundScores;
   using V = typename TR::vec;
   using E = typename TR::elem;
   constexpr int P = TR::split ? 2 : 1;
-  using FT = FlashTile<HDP, P, GM>;
-  static_assert(FT::BM == FlashTile<HDP, P, !GM>::BM, "one grid for both mask instantiations");
+  using FT = FlashTile<HDP, P>;
   constexpr int BN = FT::BN, QG = FT::QG, BM = FT::BM, NTH = FT::NTH, STAGES = FT::STAGES;
   constexpr int NC = BN / 32;          // 32-key chunks per tile
   constexpr int ND = HDP / 32;         // 32-wide contraction chunks of q . k
@@ -276,8 +260,6 @@ void flash_fwd_kernel(FlashArgs a) {
   static_assert(CV >= (HDP >= 256 ? 4 : 8) && CK >= (HDP == 32 ? 4 : HDP == 64 ? 8 : 16),
                 "K / V^T swizzle wider than a tile row");
 
-  __shared__ __attribute__((aligned(1024))) E smem[STAGES * STG];
-
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -285,13 +267,14 @@ void flash_fwd_kernel(FlashArgs a) {
 
   const int nqb = (a.S + BM - 1) / BM;
   const bool causal = a.flags & KF_FLASH_CAUSAL;
-  const FlashBlock blk = flash_block_map(blockIdx.x, gridDim.x, a.B, a.H, nqb, causal);
+  const FlashBlock blk = flash_block_map(bid, nblocks, a.B, a.H, nqb, causal);
   const int b = blk.b, h = blk.h, qb = blk.qb;
 
   const int kvlen = a.kv_len ? a.kv_len[b] : a.S;
   // prefix: keys [0, kvlen) are all valid, so kvlen alone decides validity (keep unread)
-  const bool prefix = a.keep == nullptr || (a.kv_len && a.prefix && a.prefix[b] != 0);
-  if (prefix == GM) return;            // the other instantiation serves this batch row
+  const bool is_general = a.keep && !(a.kv_len && a.prefix && a.prefix[b] != 0);
+  if (GEN ? a.only_general && !is_general : is_general) return;
+  const bool general = GEN && is_general;
   const bool skip_pad = (a.flags & KF_FLASH_SKIP_PAD_ROWS) && a.kv_len;
 
   const int q_lo = qb * BM;
@@ -434,6 +417,15 @@ void flash_fwd_kernel(FlashArgs a) {
     for (int j = 0; j < NT; ++j) acc[qg][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
 
+  // general rows: the keep value of one key of the next tile per lane
+  auto keep_of = [&](int t) KF_INLINE {
+    const int key = min(t * BN + (lane & (BN - 1)), a.S - 1);
+    return ld_elem(a.keep, a.keep_dtype, (int64_t)b * a.ld_keep + key);
+  };
+  float keep_next = 1.0f;
+  if (general && ntiles > 0) keep_next = keep_of(0);
+  uint64_t valid = 0;                  // bit i: key t * BN + i of a general row is kept
+
   for (int t = 0; t < ntiles; ++t) {
     // this wavefront's copies of tile t have landed once at most the later tiles' copies
     // are pending (loads complete in issue order; keep reads issued later only make the
@@ -450,9 +442,15 @@ void flash_fwd_kernel(FlashArgs a) {
       wait_vmcnt<0>();
     }
     lds_barrier();                   // everyone's copies landed; tile t-1 no longer read
+    if (general) {                   // ahead of the copies, so that its wait is not theirs
+      valid = __ballot(keep_next != 0.0f);
+      if (t + 1 < ntiles) keep_next = keep_of(t + 1);
+    }
     if (t + STAGES - 1 < ntiles) issue(t + STAGES - 1);
     const E* st = smem + (t % STAGES) * STG;
     const int k0 = t * BN;
+    // bit jj: key 32 c + 8 grp + jj of the tile
+    auto keep_bits = [&](int c) KF_INLINE { return (uint32_t)(valid >> (32 * c)) >> (8 * grp); };
 
     if (wave_active && k0 < kend_w) {
       if constexpr (kPipe) {
@@ -481,7 +479,7 @@ void flash_fwd_kernel(FlashArgs a) {
         auto soft1 = [&](int qg) KF_INLINE {
           const int qg0 = qw0 + qg * 16;
           const int qi = qg0 + r;
-          const bool full = !GM && k0 + BN <= kvlen && (!causal || k0 + BN - 1 <= qg0);
+          const bool full = !general && k0 + BN <= kvlen && (!causal || k0 + BN - 1 <= qg0);
 #pragma unroll
           for (int c = 0; c < NC; ++c)
 #pragma unroll
@@ -502,14 +500,12 @@ void flash_fwd_kernel(FlashArgs a) {
                 const bool ok = key < kvlen && (!causal || key <= qi);
                 x[qg][c][jj] = ok ? x[qg][c][jj] : kNegInf;
               }
-            if constexpr (GM) {
+            if (general) {
 #pragma unroll
-              for (int c = 0; c < NC; ++c) {
-                float kv[8];
-                load_keep8(a, (int64_t)b * a.ld_keep, k0 + 32 * c + 8 * grp, kv);
+              for (int c = 0; c < NC; ++c)
 #pragma unroll
-                for (int jj = 0; jj < 8; ++jj) x[qg][c][jj] = kv[jj] != 0.0f ? x[qg][c][jj] : kNegInf;
-              }
+                for (int jj = 0; jj < 8; ++jj)
+                  x[qg][c][jj] = (keep_bits(c) >> jj) & 1 ? x[qg][c][jj] : kNegInf;
             }
           }
           float mloc = kNegInf;
@@ -628,7 +624,7 @@ void flash_fwd_kernel(FlashArgs a) {
         // reads wait once per phase and V^T lands under the softmax. (The copies are
         // FLAT-encoded LDS writes, so each LDS-read wait is a wait for all reads: read
         // one fragment ahead, the MFMAs had waited for each read in turn.)
-        constexpr bool kBatch = !TR::split && QG == 1 && HDP == 256 && !GM;
+        constexpr bool kBatch = !TR::split && QG == 1 && HDP == 256;
         V kall[kBatch ? NC : 1][2][kBatch ? ND : 1];
         V vall[kBatch ? NC : 1][kBatch ? NT : 1];
         if constexpr (kBatch) {
@@ -678,7 +674,7 @@ void flash_fwd_kernel(FlashArgs a) {
         for (int qg = 0; qg < QG; ++qg) {
           const int qg0 = qw0 + qg * 16;
           const int qi = qg0 + r;
-          const bool full = !GM && k0 + BN <= kvlen && (!causal || k0 + BN - 1 <= qg0);
+          const bool full = !general && k0 + BN <= kvlen && (!causal || k0 + BN - 1 <= qg0);
           float x[NC][8];
 #pragma unroll
           for (int c = 0; c < NC; ++c)
@@ -700,14 +696,12 @@ void flash_fwd_kernel(FlashArgs a) {
                 const bool ok = key < kvlen && (!causal || key <= qi);
                 x[c][jj] = ok ? x[c][jj] : kNegInf;
               }
-            if constexpr (GM) {
+            if (general) {
 #pragma unroll
-              for (int c = 0; c < NC; ++c) {
-                float kv[8];
-                load_keep8(a, (int64_t)b * a.ld_keep, k0 + 32 * c + 8 * grp, kv);
+              for (int c = 0; c < NC; ++c)
 #pragma unroll
-                for (int jj = 0; jj < 8; ++jj) x[c][jj] = kv[jj] != 0.0f ? x[c][jj] : kNegInf;
-              }
+                for (int jj = 0; jj < 8; ++jj)
+                  x[c][jj] = (keep_bits(c) >> jj) & 1 ? x[c][jj] : kNegInf;
             }
           }
           // Lazy rescaling: p = exp2(s - m_ref) with a reference maximum that moves only
@@ -799,6 +793,53 @@ void flash_fwd_kernel(FlashArgs a) {
       float o[4] = {acc[qg][j][0] * inv, acc[qg][j][1] * inv, acc[qg][j][2] * inv, acc[qg][j][3] * inv};
       store_o4(a, obase + (int64_t)qi * a.os2 + d, o);
     }
+  }
+}
+
+template <int MODE, int HDP> constexpr int flash_stage_elems() {
+  using FT = FlashTile<HDP, ModeTraits<MODE>::split ? 2 : 1>;
+  return FT::STAGES * FT::STAGE_BYTES / 2;
+}
+
+// Wavefronts per SIMD the kernel is compiled to fit: head_dim <= 32 with single-plane P sits
+// at the 128 registers that four of them allow.
+template <int MODE, int HDP, int VAR> constexpr int flash_waves_per_simd() {
+  return HDP == 32 && MODE == MODE_F16X3 && VAR == kVarP16 ? 4 : 1;
+}
+
+// One kernel for prefix and general rows, except head_dim 128 in the split modes: there the
+// kernel is at its 256 registers, and the mask code costs the prefix rows 2 % (4 x 8 heads of
+// 1001 keys 104.8 -> 107.2 us), so the general rows take a launch of their own.
+template <int MODE, int HDP> constexpr bool flash_serves_all() {
+  return !(HDP == 128 && ModeTraits<MODE>::split);
+}
+
+template <int MODE, int QT, int HDP, int VAR = kVarNone>
+__global__ __launch_bounds__((FlashTile<HDP, ModeTraits<MODE>::split ? 2 : 1>::NTH))
+__attribute__((amdgpu_waves_per_eu(flash_waves_per_simd<MODE, HDP, VAR>())))
+void flash_fwd_kernel(FlashArgs a) {
+  __shared__ __attribute__((aligned(1024)))
+  typename ModeTraits<MODE>::elem smem[flash_stage_elems<MODE, HDP>()];
+  flash_fwd_block<MODE, QT, HDP, VAR, flash_serves_all<MODE, HDP>()>(a, blockIdx.x, gridDim.x, smem);
+}
+
+// The rows whose mask is no prefix, beside a kernel that serves the prefix ones (head_dim 8
+// packed, pipelined single pass). A few blocks a CU walk the `nblocks` of the grid, and leave
+// at once where the batch has no such row, which is the usual case: a launch of the whole
+// grid to find that out took 45 us over 32768 blocks.
+template <int MODE, int QT, int HDP, int VAR = kVarNone>
+__global__ __launch_bounds__((FlashTile<HDP, ModeTraits<MODE>::split ? 2 : 1>::NTH))
+void flash_general_kernel(FlashArgs a, int nblocks) {
+  __shared__ __attribute__((aligned(1024)))
+  typename ModeTraits<MODE>::elem smem[flash_stage_elems<MODE, HDP>()];
+  if (a.kv_len && a.prefix) {
+    int any = 0;
+    for (int b = threadIdx.x; b < a.B; b += blockDim.x) any |= a.prefix[b] == 0;
+    if (!__syncthreads_or(any)) return;
+  }
+  for (int bid = blockIdx.x; bid < nblocks; bid += gridDim.x) {
+    flash_fwd_block<MODE, QT, HDP, VAR, true>(a, bid, nblocks, smem);
+    lds_barrier();                     // the stages are read before the next block's copies
   }
 }
 
@@ -2251,77 +2292,69 @@ __global__ __launch_bounds__(SmallTile::NTH) void flash_small_kernel(FlashArgs a
   store_out(o4);
 }
 
+// The general rows of a launch whose prefix rows another kernel serves (all rows are
+// general where the extents are not given).
+template <int MODE, int QT, int HDP, int VAR = kVarNone>
+static void launch_general(FlashArgs a, hipStream_t st) {
+  if (a.keep == nullptr) return;
+  using FT = FlashTile<HDP, ModeTraits<MODE>::split ? 2 : 1>;
+  const int64_t blocks = (int64_t)((a.S + FT::BM - 1) / FT::BM) * a.B * a.H;
+  const int64_t resident = 4LL * cu_count();
+  a.only_general = 1;
+  hipLaunchKernelGGL((flash_general_kernel<MODE, QT, HDP, VAR>),
+                     dim3((unsigned)(blocks < resident ? blocks : resident)), dim3(FT::NTH), 0, st, a,
+                     (int)blocks);
+}
+
+template <int MODE, int QT, int HDP, int VAR = kVarNone>
+static void launch_fwd(const FlashArgs& a, hipStream_t st) {
+  using FT = FlashTile<HDP, ModeTraits<MODE>::split ? 2 : 1>;
+  constexpr bool all = flash_serves_all<MODE, HDP>();
+  const int64_t blocks = (int64_t)((a.S + FT::BM - 1) / FT::BM) * a.B * a.H;
+  if (all || a.keep == nullptr || (a.kv_len && a.prefix))
+    hipLaunchKernelGGL((flash_fwd_kernel<MODE, QT, HDP, VAR>), dim3((unsigned)blocks), dim3(FT::NTH), 0, st, a);
+  if constexpr (!all) launch_general<MODE, QT, HDP, VAR>(a, st);
+}
+
 template <int MODE, int QT, int HDP>
 static void launch_flash(const FlashArgs& a, hipStream_t st) {
-  using FT = FlashTile<HDP, ModeTraits<MODE>::split ? 2 : 1>;
-  using FTG = FlashTile<HDP, ModeTraits<MODE>::split ? 2 : 1, true>;   // general-mask launch
-  const int nqb = (a.S + FT::BM - 1) / FT::BM;
-  const int64_t blocks = (int64_t)nqb * a.B * a.H;
   const bool any_prefix = a.keep == nullptr || (a.kv_len && a.prefix);
-  const bool any_general = a.keep != nullptr;
   if constexpr (HDP == 32 && ModeTraits<MODE>::split) {
     // head_dim 8 in the split modes: the packed-contraction kernel for prefix-mask rows
     // (32-bit slice offsets, as the pipelined kernel), unless KF_FLASH_NO_PIPE
     const bool fits = (int64_t)a.S * a.ks2 < (1LL << 31) && (int64_t)a.hd * a.vs2 < (1LL << 31);
-    if (a.hd == SmallTile::HD && fits && !(a.flags & KF_FLASH_NO_PIPE)) {
+    if (a.hd == SmallTile::HD && fits && any_prefix && !(a.flags & KF_FLASH_NO_PIPE)) {
+      const dim3 grid((unsigned)(((a.S + SmallTile::BM - 1) / SmallTile::BM) * (int64_t)a.B * a.H));
       if constexpr (MODE == MODE_F16X3) {
         if (a.flags & KF_FLASH_P16) {
-          if (any_prefix)
-            hipLaunchKernelGGL((flash_small_kernel<MODE, QT, kVarP16>), dim3((unsigned)blocks),
-                               dim3(SmallTile::NTH), 0, st, a);
-          if (any_general)
-            hipLaunchKernelGGL((flash_fwd_kernel<MODE, QT, HDP, true, kVarP16>), dim3((unsigned)blocks), dim3(FTG::NTH), 0, st, a);
-          return;
+          hipLaunchKernelGGL((flash_small_kernel<MODE, QT, kVarP16>), grid, dim3(SmallTile::NTH), 0, st, a);
+          return launch_general<MODE, QT, HDP, kVarP16>(a, st);
         }
       }
-      if (any_prefix)
-        hipLaunchKernelGGL((flash_small_kernel<MODE, QT, kVarNone>), dim3((unsigned)blocks),
-                           dim3(SmallTile::NTH), 0, st, a);
-      if (any_general)
-        hipLaunchKernelGGL((flash_fwd_kernel<MODE, QT, HDP, true>), dim3((unsigned)blocks), dim3(FTG::NTH), 0, st, a);
-      return;
+      hipLaunchKernelGGL((flash_small_kernel<MODE, QT, kVarNone>), grid, dim3(SmallTile::NTH), 0, st, a);
+      return launch_general<MODE, QT, HDP>(a, st);
     }
   }
   if constexpr (MODE == MODE_F16X3) {
-    if (a.flags & KF_FLASH_P16) {
-      if (any_prefix)
-        hipLaunchKernelGGL((flash_fwd_kernel<MODE, QT, HDP, false, kVarP16>), dim3((unsigned)blocks), dim3(FT::NTH), 0, st, a);
-      if (any_general)
-        hipLaunchKernelGGL((flash_fwd_kernel<MODE, QT, HDP, true, kVarP16>), dim3((unsigned)blocks), dim3(FTG::NTH), 0, st, a);
-      return;
-    }
+    if (a.flags & KF_FLASH_P16) return launch_fwd<MODE, QT, HDP, kVarP16>(a, st);
   }
   if constexpr (MODE == MODE_F16 || MODE == MODE_BF16) {
-    if (a.flags & KF_FLASH_ROUND_SCORES) {
-      if (any_prefix)
-        hipLaunchKernelGGL((flash_fwd_kernel<MODE, QT, HDP, false, kVarRoundScores>), dim3((unsigned)blocks), dim3(FT::NTH), 0, st, a);
-      if (any_general)
-        hipLaunchKernelGGL((flash_fwd_kernel<MODE, QT, HDP, true, kVarRoundScores>), dim3((unsigned)blocks), dim3(FTG::NTH), 0, st, a);
-      return;
-    }
+    if (a.flags & KF_FLASH_ROUND_SCORES) return launch_fwd<MODE, QT, HDP, kVarRoundScores>(a, st);
   }
   if constexpr ((MODE == MODE_F16 || MODE == MODE_BF16) && (HDP == 64 || HDP == 128)) {
     // the pipelined kernels copy from one (batch, head) slice of K and V^T with 32-bit byte
     // offsets
     const bool fits = (int64_t)a.S * a.ks2 * 2 < (1LL << 31) && (int64_t)a.hd * a.vs2 * 2 < (1LL << 31);
-    const int64_t pipe_blocks = (int64_t)((a.S + PipeTile<HDP>::BM - 1) / PipeTile<HDP>::BM) * a.B * a.H;
-    const int64_t pair_blocks = (int64_t)((a.S + PairTile::BM - 1) / PairTile::BM) * a.B * a.H;
-    const bool pair = HDP == 64 && !(a.flags & KF_FLASH_ONE_TILE);
     if (any_prefix && fits && !(a.flags & KF_FLASH_NO_PIPE)) {
-      if (pair)
-        hipLaunchKernelGGL((flash_pair_kernel<MODE, QT>), dim3((unsigned)pair_blocks),
-                           dim3(PairTile::NTH), 0, st, a);
-      else
-        hipLaunchKernelGGL((flash_pipe_kernel<MODE, QT, HDP>), dim3((unsigned)pipe_blocks),
-                           dim3(PipeTile<HDP>::NTH), 0, st, a);
-    } else if (any_prefix)
-      hipLaunchKernelGGL((flash_fwd_kernel<MODE, QT, HDP, false>), dim3((unsigned)blocks), dim3(FT::NTH), 0, st, a);
-  } else {
-    if (any_prefix)
-      hipLaunchKernelGGL((flash_fwd_kernel<MODE, QT, HDP, false>), dim3((unsigned)blocks), dim3(FT::NTH), 0, st, a);
+      const bool pair = HDP == 64 && !(a.flags & KF_FLASH_ONE_TILE);
+      const int bm = pair ? PairTile::BM : PipeTile<HDP>::BM;
+      const dim3 grid((unsigned)(((a.S + bm - 1) / bm) * (int64_t)a.B * a.H));
+      if (pair) hipLaunchKernelGGL((flash_pair_kernel<MODE, QT>), grid, dim3(PairTile::NTH), 0, st, a);
+      else hipLaunchKernelGGL((flash_pipe_kernel<MODE, QT, HDP>), grid, dim3(PipeTile<HDP>::NTH), 0, st, a);
+      return launch_general<MODE, QT, HDP>(a, st);
+    }
   }
-  if (any_general)
-    hipLaunchKernelGGL((flash_fwd_kernel<MODE, QT, HDP, true>), dim3((unsigned)blocks), dim3(FTG::NTH), 0, st, a);
+  launch_fwd<MODE, QT, HDP>(a, st);
 }
 
 template <int MODE, int QT>

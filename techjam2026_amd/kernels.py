@@ -730,10 +730,10 @@ def flash_attention_ops(ops: AttnOperands, keep: Optional[torch.Tensor] = None,
     flags = ((L.FLASH_CAUSAL if causal else 0) | (L.FLASH_SKIP_PAD_ROWS if skip_pad_rows else 0)
              | (L.FLASH_P16 if p16 and ops.mode == L.MMA_F16X3 else 0)
              | (L.FLASH_ROUND_SCORES if round_scores else 0))
-    # kf_flash_fwd launches the prefix-mask kernel and, when a keep mask is given, the
-    # general-mask one
-    n_disp = int(keep_u8 is None or (kv_len is not None and prefix is not None)) \
-        + int(keep_u8 is not None)
+    # one kernel, and where it serves prefix masks only (head_dim 8 and 128 in the split
+    # modes, pipelined single pass) a second one for the other rows of a keep mask
+    n_disp = 1 + int(keep_u8 is not None and (
+        Dh in (8, 128) if ops.mode in SPLIT_MODES else Dh in (64, 128) and not round_scores))
     # algorithmic bytes: q, K and V^T read once, o written once (each plane it carries)
     nbytes = float(B * H * S * Dh) * (
         q.element_size() + ops.k_hi.element_size() * (2 if ops.k_lo is not None else 1)
