@@ -46,48 +46,78 @@ __global__ __launch_bounds__(256) void mask_prep_kernel(const void* keep, int dt
   }
 }
 
-// k, v [B, H, S, hd] (any strides, unit d) -> K planes (layout of ko strides) and V^T
-// planes [.., hd, keys]. One thread per 8-element chunk of one (b, h, s) row.
-template <int IT>
-__global__ __launch_bounds__(256) void attn_prep_kernel(
-    const void* k, int64_t ks0, int64_t ks1, int64_t ks2,
-    const void* v, int64_t vs0, int64_t vs1, int64_t vs2,
-    void* k_hi, void* k_lo, int64_t os0, int64_t os1, int64_t os2,
-    void* vt_hi, void* vt_lo, int64_t ts0, int64_t ts1, int64_t ts2,
-    int B, int H, int S, int hd, int kv_dtype) {
-  const int cpr = hd / 8;
-  const int64_t total = (int64_t)B * H * S * cpr;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const int c = (int)(i % cpr);
-    int64_t rest = i / cpr;
-    const int s = (int)(rest % S); rest /= S;
-    const int h = (int)(rest % H);
-    const int b = (int)(rest / H);
-    const int d = c * 8;
-    float x[8];
-    if (k_hi) {                 // null: the caller's K already has the kernel's layout
-      ld8<IT>(k, b * ks0 + h * ks1 + s * ks2 + d, x);
-      const int64_t ko = b * os0 + h * os1 + s * os2 + d;
-      store4_any(k_hi, k_lo, kv_dtype, ko, x);
-      store4_any(k_hi, k_lo, kv_dtype, ko + 4, x + 4);
-    }
-    ld8<IT>(v, b * vs0 + h * vs1 + s * vs2 + d, x);
-    const int64_t vo = b * ts0 + h * ts1 + s;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) st_elem(vt_hi, kv_dtype, vo + (int64_t)(d + e) * ts2, x[e], vt_lo);
-    if (s == S - 1) {     // zero the V^T pad columns [S, roundup(S, 8)) that attention reads
-      for (int sp = S; sp < ((S + 7) & ~7); ++sp)
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-          st_elem(vt_hi, kv_dtype, vo + (sp - s) + (int64_t)(d + e) * ts2, 0.0f, vt_lo);
-    }
-  }
-}
+// k, v [B, H, S, hd] (any strides, unit d) -> K planes (layout of ko strides) and V^T planes
+// [.., hd, keys], zero in the pad columns [S, roundup(S, 8)). HBM-bound: a thread takes an
+// 8 x 8 block (eight keys, one 8-element chunk of d) of v and turns it in registers, or the
+// same block of k. A wavefront's 64 blocks are CW chunks (whole 128-byte pieces of 16-bit rows
+// from head_dim 64) by 64 / CW key blocks, so V^T leaves in 16-byte stores that fill whole
+// lines too. One thread per key and chunk, storing its eight columns of V^T in 2-byte
+// pieces, took 65 of 1131 us of fp16 attention over 2 x 16 heads of 16384 keys (1095 now) and
+// 29.6 of 104.6 us of fp32 attention over 4 x 8 heads of 1001 keys of 128 (87.0 now).
+struct PrepArgs {
+  const void* k; int64_t ks0, ks1, ks2;
+  const void* v; int64_t vs0, vs1, vs2;
+  void* k_hi; void* k_lo; int64_t os0, os1, os2;
+  void* vt_hi; void* vt_lo; int64_t ts0, ts1, ts2;
+  int B, H, S, hd;
+  int vec_k, vec_v;        // 16-byte aligned outputs (base and strides)
+};
 
-static int kv_code(int mode) {
-  return mode == KF_MMA_F16X3 ? KF_F16X2 : mode == KF_MMA_BF16X3 ? KF_BF16X2
-       : mode == KF_MMA_F16 ? KF_F16 : KF_BF16;
+template <int IT, typename E, bool TWO>
+__global__ __launch_bounds__(256) void attn_prep_kernel(PrepArgs a) {
+  typedef E V8 __attribute__((ext_vector_type(8)));
+  const bool is_v = blockIdx.y == 0;
+  const int cpr = a.hd / 8, cw = cpr < 8 ? cpr : 8;
+  const int nsb = (a.S + 7) / 8;                     // key blocks per (b, h)
+  const int sw = 64 / cw, spans = (nsb + sw - 1) / sw, groups = cpr / cw;
+  const int lane = threadIdx.x & 63;
+  int64_t w = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (w >= (int64_t)a.B * a.H * spans * groups) return;
+  const int c = (int)(w % groups) * cw + lane % cw;
+  w /= groups;
+  const int sb = (int)(w % spans) * sw + lane / cw;
+  w /= spans;
+  const int h = (int)(w % a.H), b = (int)(w / a.H);
+  if (sb >= nsb) return;
+  const int s0 = 8 * sb, d = 8 * c;
+  const void* src = is_v ? a.v : a.k;
+  const int64_t at = is_v ? b * a.vs0 + h * a.vs1 + d : b * a.ks0 + h * a.ks1 + d;
+  const int64_t rs = is_v ? a.vs2 : a.ks2;
+  float x[8][8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) ld8<IT>(src, at + (int64_t)min(s0 + i, a.S - 1) * rs, x[i]);
+  auto put = [&](void* hi, void* lo, int64_t off, const float* v, int vec) KF_INLINE {
+    V8 p, q;
+    if constexpr (TWO) split_n<E, 8>(v, p, q);
+    else
+#pragma unroll
+      for (int e = 0; e < 8; ++e) p[e] = (E)v[e];
+    if (vec) {
+      *(V8*)((E*)hi + off) = p;
+      if constexpr (TWO) *(V8*)((E*)lo + off) = q;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        ((E*)hi)[off + e] = p[e];
+        if constexpr (TWO) ((E*)lo)[off + e] = q[e];
+      }
+    }
+  };
+  if (is_v) {
+    const int64_t o = b * a.ts0 + h * a.ts1 + s0;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      float t[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) t[i] = s0 + i < a.S ? x[i][e] : 0.0f;
+      put(a.vt_hi, a.vt_lo, o + (int64_t)(d + e) * a.ts2, t, a.vec_v);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (s0 + i < a.S)
+        put(a.k_hi, a.k_lo, b * a.os0 + h * a.os1 + (int64_t)(s0 + i) * a.os2 + d, x[i], a.vec_k);
+  }
 }
 
 }  // namespace kf
@@ -205,18 +235,27 @@ extern "C" int kf_attn_prep(const void* k, const int64_t* ks, const void* v, con
     return KF_EUNSUPPORTED;
   }
   if (B == 0 || S == 0) return KF_OK;
-  const int64_t total = B * H * S * (hd / 8);
-  int64_t blocks = (total + 255) / 256;
-  if (blocks > 65536) blocks = 65536;
-  hipStream_t st = (hipStream_t)stream;
-  const int kvd = kv_code(mode);
+  auto al16s = [](const void* hi, const void* lo, const int64_t* st) {
+    return !(((uintptr_t)hi | (uintptr_t)lo) & 15) && !((st[0] | st[1] | st[2]) & 7);
+  };
   static const int64_t zero4[4] = {0, 0, 0, 1};
   const int64_t* kst = with_k ? ks : zero4;
   const int64_t* kost = with_k ? kos : zero4;
-#define KF_PREP(IT)                                                                            \
-  hipLaunchKernelGGL(attn_prep_kernel<IT>, dim3((unsigned)blocks), dim3(256), 0, st, k, kst[0], \
-                     kst[1], kst[2], v, vs[0], vs[1], vs[2], k_hi, k_lo, kost[0], kost[1], kost[2], \
-                     vt_hi, vt_lo, vts[0], vts[1], vts[2], (int)B, (int)H, (int)S, (int)hd, kvd)
+  const int64_t cpr = hd / 8, cw = cpr < 8 ? cpr : 8, sw = 64 / cw;
+  const int64_t waves = B * H * (((S + 7) / 8 + sw - 1) / sw) * (cpr / cw);
+  if ((waves + 3) / 4 > 0x7fffffffLL) { kf_set_error("kf_attn_prep: problem too large"); return KF_EUNSUPPORTED; }
+  const dim3 grid((unsigned)((waves + 3) / 4), with_k ? 2 : 1);
+  hipStream_t st = (hipStream_t)stream;
+  const PrepArgs pa{k, kst[0], kst[1], kst[2], v, vs[0], vs[1], vs[2], k_hi, k_lo, kost[0], kost[1],
+                    kost[2], vt_hi, vt_lo, vts[0], vts[1], vts[2], (int)B, (int)H, (int)S, (int)hd,
+                    with_k && al16s(k_hi, split ? k_lo : nullptr, kos),
+                    al16s(vt_hi, split ? vt_lo : nullptr, vts)};
+  const bool bf = mode == KF_MMA_BF16 || mode == KF_MMA_BF16X3;
+#define KF_PREP(IT)                                                                                  \
+  if (bf && split) hipLaunchKernelGGL((attn_prep_kernel<IT, __bf16, true>), grid, dim3(256), 0, st, pa);  \
+  else if (bf) hipLaunchKernelGGL((attn_prep_kernel<IT, __bf16, false>), grid, dim3(256), 0, st, pa);     \
+  else if (split) hipLaunchKernelGGL((attn_prep_kernel<IT, _Float16, true>), grid, dim3(256), 0, st, pa); \
+  else hipLaunchKernelGGL((attn_prep_kernel<IT, _Float16, false>), grid, dim3(256), 0, st, pa)
   switch (in_dtype) {
     case KF_F32: KF_PREP(KF_F32); break;
     case KF_F16: KF_PREP(KF_F16); break;

@@ -1,0 +1,45 @@
+"""kf_attn_prep's eight-by-eight blocks at their edges: key counts around a block and a
+wavefront's span, every head_dim, packed and padded input rows, outputs that allow 16-byte
+stores and outputs that do not (odd V^T bases, K strides of 4): the planes are the rounded
+values bit for bit, the pad columns zero."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from techjam2026_amd import _lib as L
+from techjam2026_amd import kernels as K
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda")
+
+
+@pytest.mark.parametrize("mode", [L.MMA_F16, L.MMA_BF16, L.MMA_F16X3, L.MMA_BF16X3])
+@pytest.mark.parametrize("hd", [8, 16, 32, 64, 128, 256])
+@pytest.mark.parametrize("S", [1, 7, 8, 9, 63, 65, 130, 513])
+@pytest.mark.parametrize("odd", [False, True])
+def test_planes_are_the_rounded_values(mode, hd, S, odd):
+    B, H = 2, 3
+    dt = {L.MMA_F16: torch.float16, L.MMA_BF16: torch.bfloat16}.get(mode, torch.float32)
+    g = torch.Generator(device=DEV).manual_seed(S)
+    qkv = torch.randn(B, S, 3, H, hd, device=DEV, generator=g).to(dt)
+    k, v = (qkv[:, :, j].permute(0, 2, 1, 3) for j in (1, 2))
+    st = K.MODE_STORAGE[mode]
+    two = mode in K.SPLIT_MODES
+    sp = (S + 7) // 8 * 8
+    pad = 4 if odd else 0                       # K rows on 8-byte, V^T rows on 2-byte boundaries
+    kb = torch.full((2, B, H, S, hd + pad), 7.0, dtype=st, device=DEV)
+    vb = torch.full((2, B, H, hd, sp + (1 if odd else 0)), 7.0, dtype=st, device=DEV)
+    code = {torch.float32: L.F32, torch.float16: L.F16, torch.bfloat16: L.BF16}[dt]
+    L.check("kf_attn_prep", L.lib().kf_attn_prep(
+        k.data_ptr(), L.strides4(k), v.data_ptr(), L.strides4(v), code,
+        kb[0].data_ptr(), kb[1].data_ptr() if two else None, L.strides4(kb[0]),
+        vb[0].data_ptr(), vb[1].data_ptr() if two else None, L.strides4(vb[0]),
+        B, H, S, hd, mode, torch.cuda.current_stream().cuda_stream))
+    for out, x in ((kb[..., :hd], k), (vb[..., :S], v.transpose(-2, -1))):
+        hi = x.to(st)
+        assert torch.equal(out[0], hi)
+        if two:
+            assert torch.equal(out[1], (x.float() - hi.float()).to(st))
+    assert torch.count_nonzero(vb[: 2 if two else 1, ..., S:sp]) == 0
+    assert bool((kb[..., hd:] == 7).all() and (vb[..., sp:] == 7).all()), "wrote past the rows"
