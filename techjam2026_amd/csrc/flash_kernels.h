@@ -62,14 +62,16 @@ constexpr float kNegInf = -__builtin_huge_valf();
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLazy = 8.0f;     // log2 units: probabilities stay <= 256
 
-template <int HDP, int P = 2> struct FlashTile {
+// SMALL: 64-row blocks of four wavefronts with one 16-row group each, for grids that leave CUs
+// idle at head_dim <= 32 (launch_fwd).
+template <int HDP, int P = 2, bool SMALL = false> struct FlashTile {
   // hd 64 in the split modes: eight wavefronts of one 16-row group (the same
   // 128-row block as four of two groups) at ~100-126 VGPRs, so two blocks give each SIMD
   // four wavefronts instead of two (C2-shape f16x3 attention 28.0 -> 25.3 us, outputs
   // bit-identical: each row takes the same MFMAs and softmax steps in the same order).
-  static constexpr bool kWide64 = HDP == 64 && P == 2;
+  static constexpr bool kWide64 = HDP == 64 && P == 2 && !SMALL;
   static constexpr int BN = HDP >= 256 ? 32 : 64;   // keys per LDS stage
-  static constexpr int QG = HDP >= 256 || kWide64 ? 1 : 2;   // 16-row query groups per wavefront
+  static constexpr int QG = HDP >= 256 || kWide64 || SMALL ? 1 : 2;   // 16-row query groups per wavefront
   // Measured on MI355X (B4 H16 S8192 causal): hd >= 128 gains from eight wavefronts
   // sharing each K/V tile and three stages in flight (hd 128 f16x3: 198 -> 309 TF); hd <= 64
   // runs best with two stages (two blocks per CU).
@@ -80,7 +82,8 @@ template <int HDP, int P = 2> struct FlashTile {
   // hd 256 single-pass (32-key stages of 32 KB): four stages, two tiles of copies in flight
   // (C4-shape attention 0.416 -> 0.405 ms, measured on MI355X)
   static constexpr int STAGES = (HDP >= 256 && P == 1) ? 4 : (HDP >= 128 && 3 * STAGE_BYTES <= 160 * 1024) ? 3 : 2;
-  static_assert(BM == (HDP >= 256 ? 128 : HDP >= 128 ? 256 : 128), "one block height per head dim");
+  static_assert(BM == (SMALL ? 64 : HDP == 128 ? 256 : 128), "block height per head dim");
+  static_assert(!SMALL || HDP == 32, "small blocks are built for head_dim <= 32");
 };
 
 __device__ __forceinline__ void store_o4(const FlashArgs& a, int64_t off, const float* v) {
@@ -229,7 +232,7 @@ __host__ __device__ inline FlashBlock flash_block_map(int bid, int nblocks, int 
 }
 
 // GEN: whether this instantiation serves general rows.
-template <int MODE, int QT, int HDP, int VAR, bool GEN>
+template <int MODE, int QT, int HDP, int VAR, bool GEN, bool SMALL = false>
 __device__ __forceinline__ void flash_fwd_block(const FlashArgs& a, int bid, int nblocks,
                                                 typename ModeTraits<MODE>::elem* smem) {
   using TR = ModeTraits<MODE>;
@@ -239,12 +242,12 @@ __device__ __forceinline__ void flash_fwd_block(const FlashArgs& a, int bid, int
   constexpr bool PS = VAR != kVarP16;         // P as hi + lo in split modes
   // two query groups pipelined within a tile (their K and V^T fragments held in registers
   // for both): where those fit beside the rest (head_dim <= 64)
-  constexpr bool kPipe = FlashTile<HDP, TR::split ? 2 : 1>::QG == 2 && HDP <= 64;
+  constexpr bool kPipe = FlashTile<HDP, TR::split ? 2 : 1, SMALL>::QG == 2 && HDP <= 64;
   constexpr bool RS = VAR == kVarRoundScores;
   using V = typename TR::vec;
   using E = typename TR::elem;
   constexpr int P = TR::split ? 2 : 1;
-  using FT = FlashTile<HDP, P>;
+  using FT = FlashTile<HDP, P, SMALL>;
   constexpr int BN = FT::BN, QG = FT::QG, BM = FT::BM, NTH = FT::NTH, STAGES = FT::STAGES;
   constexpr int NC = BN / 32;          // 32-key chunks per tile
   constexpr int ND = HDP / 32;         // 32-wide contraction chunks of q . k
@@ -814,13 +817,13 @@ template <int MODE, int HDP> constexpr bool flash_serves_all() {
   return !(HDP == 128 && ModeTraits<MODE>::split);
 }
 
-template <int MODE, int QT, int HDP, int VAR = kVarNone>
-__global__ __launch_bounds__((FlashTile<HDP, ModeTraits<MODE>::split ? 2 : 1>::NTH))
+template <int MODE, int QT, int HDP, int VAR = kVarNone, bool SMALL = false>
+__global__ __launch_bounds__((FlashTile<HDP, ModeTraits<MODE>::split ? 2 : 1, SMALL>::NTH))
 __attribute__((amdgpu_waves_per_eu(flash_waves_per_simd<MODE, HDP, VAR>())))
 void flash_fwd_kernel(FlashArgs a) {
   __shared__ __attribute__((aligned(1024)))
   typename ModeTraits<MODE>::elem smem[flash_stage_elems<MODE, HDP>()];
-  flash_fwd_block<MODE, QT, HDP, VAR, flash_serves_all<MODE, HDP>()>(a, blockIdx.x, gridDim.x, smem);
+  flash_fwd_block<MODE, QT, HDP, VAR, flash_serves_all<MODE, HDP>(), SMALL>(a, blockIdx.x, gridDim.x, smem);
 }
 
 // The rows whose mask is no prefix, beside a kernel that serves the prefix ones (head_dim 8
@@ -2311,6 +2314,18 @@ static void launch_fwd(const FlashArgs& a, hipStream_t st) {
   using FT = FlashTile<HDP, ModeTraits<MODE>::split ? 2 : 1>;
   constexpr bool all = flash_serves_all<MODE, HDP>();
   const int64_t blocks = (int64_t)((a.S + FT::BM - 1) / FT::BM) * a.B * a.H;
+  // Grids with fewer blocks than CUs: half the rows per block, one row group per wavefront, so
+  // twice the CUs and half the chain per wavefront (four heads of 128 keys 8.0 -> 6.0 us a
+  // launch; head_dim 64, whose wavefronts have one group already, gains nothing). Same
+  // results: a row takes the same steps in the same order.
+  if constexpr (HDP == 32) {
+    if (blocks < cu_count()) {
+      using FS = FlashTile<HDP, ModeTraits<MODE>::split ? 2 : 1, true>;
+      const int64_t small = (int64_t)((a.S + FS::BM - 1) / FS::BM) * a.B * a.H;
+      hipLaunchKernelGGL((flash_fwd_kernel<MODE, QT, HDP, VAR, true>), dim3((unsigned)small), dim3(FS::NTH), 0, st, a);
+      return;
+    }
+  }
   if (all || a.keep == nullptr || (a.kv_len && a.prefix))
     hipLaunchKernelGGL((flash_fwd_kernel<MODE, QT, HDP, VAR>), dim3((unsigned)blocks), dim3(FT::NTH), 0, st, a);
   if constexpr (!all) launch_general<MODE, QT, HDP, VAR>(a, st);
