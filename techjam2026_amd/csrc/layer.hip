@@ -19,7 +19,7 @@
 // chain of products. Measured on MI355X against the separate kernels: a d = F = 128 layer over
 // 10000 x 128 rows (entry block, attention, tail) 4.90 -> 2.71 ms; four such layers over one
 // 128-token sequence, replayed from a graph, 206 -> 93 us; d 64, F 256, 64 x 1024 rows
-// 190 -> 130 us; d 256, F 1024, 2 x 128 rows 76 -> 57 us.
+// 190 -> 130 us; d 256, F 1024, 2 x 128 rows 76 -> 57 us (each before later changes).
 //
 // Split: a block has d / 16 / FN wavefronts, each owning 16 FN columns of every product and all
 // BM rows. The product is formed as W . A^T, so a lane holds four
@@ -158,8 +158,8 @@ void layer_kernel(LayerArgs g) {
       for (int j = 0; j < FM; ++j) c.v[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   };
   // acc += product p of the rows in `a`; fetches the group after each group as it goes
-  auto group = [&](Acc& c, const _Float16 (*a)[BM * LDA], int gk, auto PAc, auto PWc, auto SWc, auto LO)
-      KF_INLINE {
+  auto group = [&](Acc& c, const _Float16 (*a)[BM * LDA], int gk, auto Z, auto PAc, auto PWc,
+                   auto SWc, auto LO) KF_INLINE {
     constexpr int PA = decltype(PAc)::value, PW = decltype(PWc)::value;
 #pragma unroll
     for (int ks = 0; ks < C::GK; ++ks) {
@@ -175,6 +175,12 @@ void layer_kernel(LayerArgs g) {
       };
 #pragma unroll
       for (int i = 0; i < FN; ++i) {
+        // a product that starts from zero passes it to its first MFMAs
+        if constexpr (decltype(Z)::value) {
+          if (gk == 0 && ks == 0)
+#pragma unroll
+            for (int j = 0; j < FM; ++j) c.v[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
         if constexpr (PA == 2)
 #pragma unroll
           for (int j = 0; j < FM; ++j) mm(w[ks][i][0], af[j][1], c.v[i][j]);
@@ -189,24 +195,25 @@ void layer_kernel(LayerArgs g) {
   };
   using I1 = std::integral_constant<int, 1>;
   using I2 = std::integral_constant<int, 2>;
-  auto product = [&](Acc& c, const _Float16 (*a)[BM * LDA], int p, int mode, auto SWc) KF_INLINE {
+  auto product = [&](Acc& c, const _Float16 (*a)[BM * LDA], int p, int mode, auto Z, auto SWc)
+      KF_INLINE {
 #pragma unroll
     for (int gk = 0; gk < C::NG; ++gk) {
       const bool more = gk + 1 < C::NG;
       aim(more ? p : p + 1, more ? gk + 1 : 0);
       if constexpr (UNI) {
-        group(c, a, gk, I2{}, I2{}, SWc, Yes{});
+        group(c, a, gk, Z, I2{}, I2{}, SWc, Yes{});
       } else {
         const bool lo = nw_lo != nullptr;
         if (mode == KF_MMA_F16X3) {
-          if (lo) group(c, a, gk, I2{}, I2{}, SWc, Yes{});
-          else group(c, a, gk, I2{}, I2{}, SWc, No{});
+          if (lo) group(c, a, gk, Z, I2{}, I2{}, SWc, Yes{});
+          else group(c, a, gk, Z, I2{}, I2{}, SWc, No{});
         } else if (mode == KF_MMA_F16X2) {
-          if (lo) group(c, a, gk, I1{}, I2{}, SWc, Yes{});
-          else group(c, a, gk, I1{}, I2{}, SWc, No{});
+          if (lo) group(c, a, gk, Z, I1{}, I2{}, SWc, Yes{});
+          else group(c, a, gk, Z, I1{}, I2{}, SWc, No{});
         } else {
-          if (lo) group(c, a, gk, I1{}, I1{}, SWc, Yes{});
-          else group(c, a, gk, I1{}, I1{}, SWc, No{});
+          if (lo) group(c, a, gk, Z, I1{}, I1{}, SWc, Yes{});
+          else group(c, a, gk, Z, I1{}, I1{}, SWc, No{});
         }
       }
     }
@@ -285,6 +292,30 @@ void layer_kernel(LayerArgs g) {
     auto q = __builtin_amdgcn_permlane32_swap(__float_as_uint(t), __float_as_uint(t), false, false);
     return __uint_as_float(q[0]) + __uint_as_float(q[1]);
   };
+  // Two quads of adjacent tiles p and q, traded between neighbouring lane groups: each lane
+  // ends with eight consecutive values of one tile, those from offset pair8 on. Stores then
+  // leave in 16-byte pieces, a wavefront's row (or V^T column) in 64 bytes of 16-bit values
+  // instead of 32 (10000 x 128 rows of d 128: entry, attention and tail 2150 -> 1999 us).
+  auto trade = [&](const f32x4& p, const f32x4& q, float* v) KF_INLINE {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const auto t = __builtin_amdgcn_permlane16_swap(__float_as_uint(p[e]), __float_as_uint(q[e]), false, false);
+      v[e] = __uint_as_float(t[0]);
+      v[4 + e] = __uint_as_float(t[1]);
+    }
+  };
+  const int pair8 = 16 * (grp & 1) + 4 * (grp & 2);
+  // eight fp32 values, or their fp16 plane(s), at an element offset
+  auto put8 = [&](float* p, int64_t at, const float* v) KF_INLINE {
+    *(f32x4*)(p + at) = f32x4{v[0], v[1], v[2], v[3]};
+    *(f32x4*)(p + at + 4) = f32x4{v[4], v[5], v[6], v[7]};
+  };
+  auto put8h = [&](_Float16* hi_p, _Float16* lo_p, int64_t at, const float* v) KF_INLINE {
+    half8 hi, lo;
+    split_n<_Float16, 8>(v, hi, lo);
+    *(half8*)(hi_p + at) = hi;
+    if (lo_p) *(half8*)(lo_p + at) = lo;
+  };
   // (mean, M2) of this wavefront's 16-column tiles of s, per row
   auto stats_out = [&]() KF_INLINE {
     float2 t[FN][FM];
@@ -306,19 +337,36 @@ void layer_kernel(LayerArgs g) {
         for (int j = 0; j < FM; ++j) red[wave * FN + i][16 * j + r] = t[i][j];
     }
   };
-  auto stats_in = [&](int j, float eps, float& mean, float& rstd) KF_INLINE {
-    float2 t[CT];
-    float sum = 0.0f;
+  // (mean, 1 / std) of this lane's rows. The lanes of a row all need them: each column group
+  // works out its share of the FM rows and the groups exchange the results.
+  auto stats_in = [&](float eps, float (&mean)[FM], float (&rstd)[FM]) KF_INLINE {
+    constexpr int OWN = FM > 4 ? FM / 4 : 1, GRPS = FM / OWN;   // rows per group, groups used
+    static_assert(GRPS == 1 || GRPS == 2 || GRPS == 4, "rows over the four column groups");
+    float om[OWN], os[OWN];
 #pragma unroll
-    for (int n = 0; n < CT; ++n) { t[n] = red[n][16 * j + r]; sum += t[n].x; }
-    mean = sum * (1.0f / CT);
-    float m2 = 0.0f;
+    for (int o = 0; o < OWN; ++o) {
+      const int j = (grp % GRPS) * OWN + o;
+      float2 t[CT];
+      float sum = 0.0f;
 #pragma unroll
-    for (int n = 0; n < CT; ++n) {
-      const float dm = t[n].x - mean;
-      m2 += __builtin_fmaf(16.0f * dm, dm, t[n].y);
+      for (int n = 0; n < CT; ++n) { t[n] = red[n][16 * j + r]; sum += t[n].x; }
+      om[o] = sum * (1.0f / CT);
+      float m2 = 0.0f;
+#pragma unroll
+      for (int n = 0; n < CT; ++n) {
+        const float dm = t[n].x - om[o];
+        m2 += __builtin_fmaf(16.0f * dm, dm, t[n].y);
+      }
+      os[o] = 1.0f / sqrtf(__builtin_fmaf(m2, 1.0f / D, eps));
     }
-    rstd = 1.0f / sqrtf(__builtin_fmaf(m2, 1.0f / D, eps));
+#pragma unroll
+    for (int j = 0; j < FM; ++j) {
+      if constexpr (GRPS == 1) { mean[j] = om[j]; rstd[j] = os[j]; }
+      else {
+        mean[j] = __shfl(om[j % OWN], 16 * (j / OWN) + r);
+        rstd[j] = __shfl(os[j % OWN], 16 * (j / OWN) + r);
+      }
+    }
   };
   // planes of four values into an LDS operand tile
   auto put4 = [&](_Float16 (*a)[BM * LDA], int row, int col, const float* v, bool two) KF_INLINE {
@@ -329,17 +377,17 @@ void layer_kernel(LayerArgs g) {
   };
   // normalised rows: h planes into xa
   auto norm_to_lds = [&](int which, float eps, bool two) KF_INLINE {
+    float mean[FM], rstd[FM];
+    stats_in(eps, mean, rstd);
 #pragma unroll
     for (int j = 0; j < FM; ++j) {
-      float mean, rstd;
-      stats_in(j, eps, mean, rstd);
 #pragma unroll
       for (int i = 0; i < FN; ++i) {
         const f32x4 gv = param(which, i), bv = param(which + 1, i);
         float v[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          v[e] = __builtin_fmaf((s.v[i][j][e] - mean) * rstd, gv[e], bv[e]);
+          v[e] = __builtin_fmaf((s.v[i][j][e] - mean[j]) * rstd[j], gv[e], bv[e]);
         put4(xa, 16 * j + r, col0 + 16 * i + 4 * grp, v, two);
       }
     }
@@ -359,8 +407,7 @@ void layer_kernel(LayerArgs g) {
 
   if constexpr (TAIL) {
     Acc acc, out;
-    zero(out);
-    product(out, xa, 0, g.m_out, No{});
+    product(out, xa, 0, g.m_out, Yes{}, No{});
     add_rows(out, 0);
     stats_out();
     lds_barrier();                               // also: every read of ctx is done
@@ -373,8 +420,7 @@ void layer_kernel(LayerArgs g) {
 #pragma unroll
       for (int i = 0; i < FN; ++i)
         b1[i] = *(const f32x4*)(g.b1 + min(c * D + col0 + 16 * i + 4 * grp, g.F - 4));
-      zero(acc);
-      product(acc, xa, 1 + 2 * c, g.m_f1, No{});
+      product(acc, xa, 1 + 2 * c, g.m_f1, Yes{}, No{});
       if (c > 0) lds_barrier();                  // the previous chunk's reads of hid are done
 #pragma unroll
       for (int i = 0; i < FN; ++i) {
@@ -388,7 +434,7 @@ void layer_kernel(LayerArgs g) {
         }
       }
       lds_barrier();
-      product(out, hid, 2 + 2 * c, g.m_f2, No{});
+      product(out, hid, 2 + 2 * c, g.m_f2, No{}, No{});
     }
     add_rows(out, 3);
   } else {
@@ -404,29 +450,50 @@ void layer_kernel(LayerArgs g) {
 #pragma unroll
     for (int j = 0; j < FM; ++j) {
       const int m = m0 + 16 * j + r;
-      if (m < g.M)
+      if constexpr (FN == 2) {
+        float v[8];
+        trade(s.v[0][j], s.v[1][j], v);
+        if (m < g.M) put8(g.s_out, (int64_t)m * D + col0 + pair8, v);
+      } else if (m < g.M) {
 #pragma unroll
         for (int i = 0; i < FN; ++i)
           *(f32x4*)(g.s_out + (int64_t)m * D + col0 + 16 * i + 4 * grp) = s.v[i][j];
+      }
     }
   }
   stats_out();
   lds_barrier();
   if constexpr (!QKV) {
+    float mean[FM], rstd[FM];
+    stats_in(g.epsn, mean, rstd);
 #pragma unroll
     for (int j = 0; j < FM; ++j) {
-      float mean, rstd;
-      stats_in(j, g.epsn, mean, rstd);
       const int m = m0 + 16 * j + r;
+      f32x4 o[FN];
 #pragma unroll
       for (int i = 0; i < FN; ++i) {
         const f32x4 gv = param(kOwn, i), bv = param(kOwn + 1, i);
-        float v[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          v[e] = __builtin_fmaf((s.v[i][j][e] - mean) * rstd, gv[e], bv[e]) * kv[j];
-        if (m < g.M)
+          o[i][e] = __builtin_fmaf((s.v[i][j][e] - mean[j]) * rstd[j], gv[e], bv[e]) * kv[j];
+      }
+      if constexpr (FN == 2) {
+        float v[8];
+        trade(o[0], o[1], v);
+        if (m < g.M) {
+          const int64_t at = (int64_t)m * D + col0 + pair8;
+          if (g.y_dtype == KF_F32) put8((float*)g.y, at, v);
+          else {
+            store4_any(g.y, nullptr, g.y_dtype, at, v);
+            store4_any(g.y, nullptr, g.y_dtype, at + 4, v + 4);
+          }
+        }
+      } else if (m < g.M) {
+#pragma unroll
+        for (int i = 0; i < FN; ++i) {
+          const float v[4] = {o[i][0], o[i][1], o[i][2], o[i][3]};
           store4_any(g.y, nullptr, g.y_dtype, (int64_t)m * D + col0 + 16 * i + 4 * grp, v);
+        }
       }
     }
   } else {
@@ -440,51 +507,81 @@ void layer_kernel(LayerArgs g) {
       if constexpr (FM * C::KS > 8) asm volatile("" ::: "memory");
     };
     // q: fp32, token-major
-    zero(acc);
-    product(acc, xa, p_qkv, g.m_attn, No{});
+    product(acc, xa, p_qkv, g.m_attn, Yes{}, No{});
+    auto add_bias = [&](int which) KF_INLINE {
 #pragma unroll
-    for (int i = 0; i < FN; ++i) {
-      const f32x4 bv = param(kOwn + 2, i);
+      for (int i = 0; i < FN; ++i) {
+        const f32x4 bv = param(which, i);
 #pragma unroll
-      for (int j = 0; j < FM; ++j) {
-        const int m = m0 + 16 * j + r;
-        if (m < g.M)
-          *(f32x4*)(g.q_out + (int64_t)m * D + col0 + 16 * i + 4 * grp) = acc.v[i][j] + bv;
+        for (int j = 0; j < FM; ++j) acc.v[i][j] += bv;
+      }
+    };
+    add_bias(kOwn + 2);
+#pragma unroll
+    for (int j = 0; j < FM; ++j) {
+      const int m = m0 + 16 * j + r;
+      if constexpr (FN == 2) {
+        float v[8];
+        trade(acc.v[0][j], acc.v[1][j], v);
+        if (m < g.M) put8(g.q_out, (int64_t)m * D + col0 + pair8, v);
+      } else if (m < g.M) {
+#pragma unroll
+        for (int i = 0; i < FN; ++i)
+          *(f32x4*)(g.q_out + (int64_t)m * D + col0 + 16 * i + 4 * grp) = acc.v[i][j];
       }
     }
     // k: planes, token-major
     reread();
-    zero(acc);
-    product(acc, xa, p_qkv + 1, g.m_attn, No{});
+    product(acc, xa, p_qkv + 1, g.m_attn, Yes{}, No{});
+    add_bias(kOwn + 3);
 #pragma unroll
-    for (int i = 0; i < FN; ++i) {
-      const f32x4 bv = param(kOwn + 3, i);
+    for (int j = 0; j < FM; ++j) {
+      const int m = m0 + 16 * j + r;
+      if constexpr (FN == 2) {
+        float v[8];
+        trade(acc.v[0][j], acc.v[1][j], v);
+        if (m < g.M) put8h(g.k_hi, g.k_lo, (int64_t)m * D + col0 + pair8, v);
+      } else {
 #pragma unroll
-      for (int j = 0; j < FM; ++j) {
-        const int m = m0 + 16 * j + r;
-        const int64_t at = (int64_t)m * D + col0 + 16 * i + 4 * grp;
-        float v[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = acc.v[i][j][e] + bv[e];
-        half4 hi, lo;
-        split_n<_Float16, 4>(v, hi, lo);
-        if (m < g.M) {
-          *(half4*)(g.k_hi + at) = hi;
-          if (k_two) *(half4*)(g.k_lo + at) = lo;
+        for (int i = 0; i < FN; ++i) {
+          const int64_t at = (int64_t)m * D + col0 + 16 * i + 4 * grp;
+          const float v[4] = {acc.v[i][j][0], acc.v[i][j][1], acc.v[i][j][2], acc.v[i][j][3]};
+          half4 hi, lo;
+          split_n<_Float16, 4>(v, hi, lo);
+          if (m < g.M) {
+            *(half4*)(g.k_hi + at) = hi;
+            if (k_two) *(half4*)(g.k_lo + at) = lo;
+          }
         }
       }
     }
     // v^T [B, d, sp]: the operands swapped, so a lane holds tokens 4 grp .. 4 grp + 3 of
     // column r; the lane that has a sequence's last token also zeroes the pad [S, sp)
     reread();
-    zero(acc);
-    product(acc, xa, p_qkv + 2, g.m_attn, Yes{});
+    product(acc, xa, p_qkv + 2, g.m_attn, Yes{}, Yes{});
 #pragma unroll
     for (int i = 0; i < FN; ++i) {
       const int n = col0 + 16 * i + r;
       const float bv = par[(kOwn + 4) * D + n];
       _Float16* vh = g.vt_hi + (int64_t)n * g.sp;
       _Float16* vl = k_two ? g.vt_lo + (int64_t)n * g.sp : nullptr;
+      if constexpr (FM % 2 == 0) {
+        if (g.S % 8 == 0) {                      // eight tokens are of one sequence; no padding
+#pragma unroll
+          for (int j = 0; j < FM; j += 2) {
+            float v[8];
+            trade(acc.v[i][j], acc.v[i][j + 1], v);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] += bv;
+            const int m = m0 + 16 * j + pair8;
+            if (m < g.M) {
+              const int b = m / g.S, t = m - b * g.S;
+              put8h(vh, vl, (int64_t)b * D * g.sp + t, v);
+            }
+          }
+          continue;
+        }
+      }
 #pragma unroll
       for (int j = 0; j < FM; ++j) {
         const int m = m0 + 16 * j + 4 * grp;
@@ -556,9 +653,9 @@ static void launch_role(const LayerArgs& a, int role, bool uni, hipStream_t st) 
 
 // Rows per block. Few rows a block while the grid does not fill the chip (the chain of
 // products of one block is the launch time), more where it does (a block reads every weight
-// once). Measured on MI355X, tail + QKV, f16x3, F = d, 16 / 32 / 64 rows: d 128 M 8192 16.0 / 14.3
-// / 23.0 us, M 65536 104 / 80 / 71; d 256 M 8192 47 / 34 / 50, M 65536 400 / 280 / 239; d 64
-// (F 256) M 8192 10.4 / 11.5 / 17.8, M 65536 52 / 42 / 46; d 32 M 8192 5.4 / 6.5 / 9.1. The
+// once). Measured on MI355X, tail + QKV, f16x3, F = d, 16 / 32 / 64 rows: d 128 M 8192 15.4 / 13.3
+// / 20.2 us, M 65536 103 / 74 / 62; d 256 M 8192 45 / 31 / 43, M 65536 389 / 259 / 218; d 64
+// (F 256) M 8192 10.6 / 11.3, M 65536 52 / 40; d 32 M 8192 5.5 / 6.1, M 65536 14.5 / 13.4. The
 // 64-row block gives a wavefront two column tiles (half the LDS reads per product; 4 wavefronts
 // a block at d 128) and needs the registers of the single-mode kernel: with stage modes read
 // at run time it spills, and widths up to 64 gain nothing from it, so those keep 32.
@@ -574,7 +671,6 @@ static void launch_d(const LayerArgs& a, int role, int rows, bool uni, hipStream
 }
 
 static inline bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
-static inline bool al8(const void* p) { return ((uintptr_t)p & 7) == 0; }
 static bool mode_ok(int m) { return m == KF_MMA_F16 || m == KF_MMA_F16X2 || m == KF_MMA_F16X3; }
 // a stage's operands: 16-byte aligned weight planes (lo where the mode has one) and bias
 static bool stage_ok(int m, const void* hi, const void* lo, const void* bias) {
@@ -658,7 +754,7 @@ extern "C" int kf_layer_block(const kf_layer_args* p, void* stream) {
       return KF_EINVAL;
     }
     if (!stage_ok(p->attn_mode, p->wqkv_hi, p->wqkv_lo, p->bqkv) || !al16(p->q_out) ||
-        !al8(p->k_hi) || !al8(p->vt_hi) || (p->k_lo && (!al8(p->k_lo) || !al8(p->vt_lo)))) {
+        !al16(p->k_hi) || !al16(p->vt_hi) || (p->k_lo && (!al16(p->k_lo) || !al16(p->vt_lo)))) {
       kf_set_error("kf_layer_block: unsupported qkv operands (mode %d)", p->attn_mode);
       return KF_EUNSUPPORTED;
     }
