@@ -62,8 +62,8 @@ constexpr float kNegInf = -__builtin_huge_valf();
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLazy = 8.0f;     // log2 units: probabilities stay <= 256
 
-// SMALL: 64-row blocks of four wavefronts with one 16-row group each, for grids that leave CUs
-// idle at head_dim <= 32 (launch_fwd).
+// SMALL: one 16-row group per wavefront instead of two (64-row blocks of four wavefronts at
+// head_dim <= 32, 128-row blocks of eight at 128), for grids that leave CUs idle (launch_fwd).
 template <int HDP, int P = 2, bool SMALL = false> struct FlashTile {
   // hd 64 in the split modes: eight wavefronts of one 16-row group (the same
   // 128-row block as four of two groups) at ~100-126 VGPRs, so two blocks give each SIMD
@@ -82,8 +82,8 @@ template <int HDP, int P = 2, bool SMALL = false> struct FlashTile {
   // hd 256 single-pass (32-key stages of 32 KB): four stages, two tiles of copies in flight
   // (C4-shape attention 0.416 -> 0.405 ms, measured on MI355X)
   static constexpr int STAGES = (HDP >= 256 && P == 1) ? 4 : (HDP >= 128 && 3 * STAGE_BYTES <= 160 * 1024) ? 3 : 2;
-  static_assert(BM == (SMALL ? 64 : HDP == 128 ? 256 : 128), "block height per head dim");
-  static_assert(!SMALL || HDP == 32, "small blocks are built for head_dim <= 32");
+  static_assert(BM == (HDP == 128 ? 256 : 128) / (SMALL ? 2 : 1), "block height per head dim");
+  static_assert(!SMALL || HDP == 32 || HDP == 128, "head dims with small blocks");
 };
 
 __device__ __forceinline__ void store_o4(const FlashArgs& a, int64_t off, const float* v) {
@@ -2314,19 +2314,23 @@ static void launch_fwd(const FlashArgs& a, hipStream_t st) {
   using FT = FlashTile<HDP, ModeTraits<MODE>::split ? 2 : 1>;
   constexpr bool all = flash_serves_all<MODE, HDP>();
   const int64_t blocks = (int64_t)((a.S + FT::BM - 1) / FT::BM) * a.B * a.H;
-  // Grids with fewer blocks than CUs: half the rows per block, one row group per wavefront, so
-  // twice the CUs and half the chain per wavefront (four heads of 128 keys 8.0 -> 6.0 us a
-  // launch; head_dim 64, whose wavefronts have one group already, gains nothing). Same
+  // Grids that leave CUs idle: half the rows per block, one row group per wavefront, so
+  // twice the CUs and half the chain per wavefront (head_dim 32, four heads of 128 keys:
+  // 8.0 -> 6.0 us a launch; head_dim 128, 32 heads of 1001 keys, f16x3: 87.2 -> 64.5 us with
+  // the preparation). At head_dim 128 a block fills a CU, so half-height blocks pay only where
+  // all of them run at once; head_dim 64 and 256 have one group a wavefront already. Same
   // results: a row takes the same steps in the same order.
-  if constexpr (HDP == 32) {
-    if (blocks < cu_count()) {
+  const bool prefix_rows = all || a.keep == nullptr || (a.kv_len && a.prefix);
+  if constexpr (HDP == 32 || (HDP == 128 && ModeTraits<MODE>::split)) {
+    if (prefix_rows && blocks * (HDP == 128 ? 2 : 1) <= cu_count()) {
       using FS = FlashTile<HDP, ModeTraits<MODE>::split ? 2 : 1, true>;
       const int64_t small = (int64_t)((a.S + FS::BM - 1) / FS::BM) * a.B * a.H;
       hipLaunchKernelGGL((flash_fwd_kernel<MODE, QT, HDP, VAR, true>), dim3((unsigned)small), dim3(FS::NTH), 0, st, a);
+      if constexpr (!all) launch_general<MODE, QT, HDP, VAR>(a, st);
       return;
     }
   }
-  if (all || a.keep == nullptr || (a.kv_len && a.prefix))
+  if (prefix_rows)
     hipLaunchKernelGGL((flash_fwd_kernel<MODE, QT, HDP, VAR>), dim3((unsigned)blocks), dim3(FT::NTH), 0, st, a);
   if constexpr (!all) launch_general<MODE, QT, HDP, VAR>(a, st);
 }
