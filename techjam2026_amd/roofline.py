@@ -189,7 +189,7 @@ def copy_calibration(mbytes: int = 1024, repeats: int = 5) -> None:
 
 # kernel-name fragment each wrapper label's dispatches must carry
 _LABEL_KERNEL = {"gemm": "gemm", "gemm_qkv": "gemm", "flash": "kf::flash_", "add_mask_ln": "ln_rows",
-                 "mask_prep": "mask_prep", "split": "split"}
+                 "mask_prep": "mask_prep", "split": "split", "layer_block": "layer_kernel"}
 
 
 def _counter_rows(directory: str, counter: str):
