@@ -589,7 +589,8 @@ class LayerBlock:
         self.work = (f"layer_block[{M}x{d}]", flops, nbytes)
 
     def __call__(self, res: torch.Tensor):
-        a = self.args
+        # a copy: another thread's call can't change the pointers between here and the launch
+        a = L.LayerArgs.from_buffer_copy(self.args)
         assert res.is_cuda and res.dtype == torch.float32 and tuple(res.shape) == (a.M, a.d) \
             and res.stride(1) == 1
         a.res, a.ld_res = res.data_ptr(), res.stride(0)
