@@ -353,9 +353,8 @@ class FusedTransformer(BaselineTransformer):
         res = x.reshape(M, d)
         if p.io_dtype != torch.float32:      # 16-bit input: widened once, fp32 inside
             res = res.float()
+        res = _entry_rows(res)
         if p.narrow:
-            if res.stride(1) != 1 or res.stride(0) % 4 or res.data_ptr() % 16:
-                res = res.clone(memory_format=torch.contiguous_format)
             if p.entry is None:
                 # the first residual is x itself (the row kernel applies the mask where it
                 # reads it), unless a captured layer reads it
@@ -477,6 +476,18 @@ class FusedTransformer(BaselineTransformer):
             runner = kind(self, x, valid_token_mask)
             self._graphs[key] = runner
         return runner(self, x, valid_token_mask)
+
+
+def _entry_rows(rows: torch.Tensor) -> torch.Tensor:
+    """Rows that the entry kernels read in 16-byte pieces: [M, d] itself, or a dense copy where
+    rows overlap or repeat (x expanded over the batch or the sequence, frames of a signal: the
+    kernels take row strides of at least d), are not of unit stride or are not 16-byte aligned
+    (16384 unaligned rows of d 1024, one layer: 1110 us a forward copied, 1165 through the unaligned
+    LayerNorm path)."""
+    if (rows.stride(1) == 1 and rows.stride(0) >= rows.shape[1] and rows.stride(0) % 4 == 0
+            and rows.data_ptr() % 16 == 0):
+        return rows
+    return rows.clone(memory_format=torch.contiguous_format)
 
 
 def _norm_of(ln):

@@ -39,3 +39,35 @@ def test_replays_equal_the_eager_forward(d, H, F, layers, mask):
     assert len(graphed._graphs) == 1
     for i, (got, want) in enumerate(held):
         assert torch.equal(got, want), f"call {i}"
+
+
+def _x_forms(B, S, d, g):
+    """[B, S, d] inputs whose rows overlap or repeat, with the dense tensor of the same values."""
+    signal = torch.randn(16 * S + d, device=DEV, generator=g)
+    token = torch.randn(1, 1, d, device=DEV, generator=g)
+    seq = torch.randn(1, S, d, device=DEV, generator=g)
+    forms = {"sequence expanded over the batch": seq.expand(B, S, d)}
+    if B == 1:
+        forms["token expanded over the sequence"] = token.expand(1, S, d)
+        forms["frames, hop 16"] = signal.unfold(0, d, 16)[:S][None]
+        forms["frames, hop 3"] = signal.unfold(0, d, 3)[:S][None]
+        if S == 1:
+            forms["one row of stride 0"] = token.expand(1, 5, d)[:, :1]
+    return forms
+
+
+@pytest.mark.parametrize("d,H,F,layers", [(128, 4, 192, 1), (64, 8, 64, 2), (512, 8, 512, 2)])
+@pytest.mark.parametrize("B,S", [(1, 45), (1, 1), (3, 45)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_rows_that_overlap_or_repeat(d, H, F, layers, B, S, dtype):
+    base = make_model(TransformerConfig(B, S, d, H, F, layers, True), device=DEV)
+    graphed = build_shared(base.config, LADDER["graph"], base)
+    g = torch.Generator(device=DEV).manual_seed(2)
+    with torch.inference_mode():
+        for what, x in _x_forms(B, S, d, g).items():
+            x = x.to(dtype) if dtype != torch.float32 else x
+            dense = x.contiguous().clone(memory_format=torch.contiguous_format)
+            for form in (x, dense, x):
+                got = graphed(form, None)
+                want = build_shared(base.config, LADDER["f16x3"], base)(dense, None)
+                assert torch.equal(got, want), what

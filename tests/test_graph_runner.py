@@ -1,0 +1,33 @@
+"""The graph path's host side on the CPU: which inputs reach the entry kernels as they are."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from techjam2026_amd.optimized import _entry_rows
+
+D, S = 32, 12
+
+
+@pytest.mark.parametrize("make,as_is", [
+    (lambda t: t[: S * D].view(S, D), True),
+    (lambda t: t[: 2 * S * D].view(S, 2 * D)[:, :D], True),         # rows of a wider tensor
+    (lambda t: t[4: 4 + S * D].view(S, D), True),
+    (lambda t: t[1: 1 + S * D].view(S, D), False),                  # 4-byte aligned
+    (lambda t: t[: S * (D + 2)].view(S, D + 2)[:, :D], False),      # every other row aligned
+    (lambda t: t[: 2 * S * D].view(S, 2 * D)[:, ::2], False),
+    (lambda t: t[: S * D].view(D, S).t(), False),
+    (lambda t: t[:D].expand(S, D), False),                          # one row repeated
+    (lambda t: t.unfold(0, D, 16)[:S], False),                      # overlapping frames
+    (lambda t: t.unfold(0, D, 4)[:S], False),
+    (lambda t: t[:D].expand(5, D)[:1], False),                      # one row of stride 0
+])
+def test_entry_rows_are_dense_and_aligned(make, as_is):
+    storage = torch.randn(4 * S * D)
+    assert storage.data_ptr() % 16 == 0
+    rows = make(storage)
+    got = _entry_rows(rows)
+    assert torch.equal(got, rows)
+    assert (got.data_ptr() == rows.data_ptr()) == as_is
+    assert got.stride(1) == 1 and got.stride(0) >= D
+    assert got.stride(0) % 4 == 0 and got.data_ptr() % 16 == 0
