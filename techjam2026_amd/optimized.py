@@ -31,6 +31,7 @@ after the final norm.
 from __future__ import annotations
 
 import dataclasses
+import threading
 from typing import Dict, List, Optional, Tuple
 
 import torch
@@ -298,9 +299,9 @@ class FusedTransformer(BaselineTransformer):
     def _eager_forward(self, x: torch.Tensor,
                        valid_token_mask: Optional[torch.Tensor]) -> torch.Tensor:
         p = self._plan_pass(x, valid_token_mask)
-        self._enter(p, x)
+        p.res = self._enter(p, x)
         self._layer_steps(p)
-        return self._leave(p)
+        return self._leave(p, p.res)
 
     # A forward in three parts: `_enter` launches the kernel that reads x, `_layer_steps`
     # everything between, `_leave` the kernel that writes the output. `GraphRunner` captures
@@ -346,9 +347,11 @@ class FusedTransformer(BaselineTransformer):
                      h_ffn=K.planes_format(m_f1), hid_fmt=K.planes_format(m_f2),
                      narrow=self._rows_fused(rdtype, modes), keep2d=keep2d)
 
-    def _enter(self, p: "_Pass", x: torch.Tensor, into_graph: bool = False) -> None:
-        """The entry LayerNorm (narrow models: with the first q, k, v^T). `into_graph`: the
-        outputs are the graph's inputs, buffers of their own, written again by each call."""
+    def _enter(self, p: "_Pass", x: torch.Tensor, into_graph: bool = False) -> torch.Tensor:
+        """The entry LayerNorm (narrow models: with the first q, k, v^T); returns the residual
+        rows. `into_graph`: the outputs are the graph's inputs, buffers of their own, written
+        again by each call; rows that no captured layer reads are the caller's own, and `p`
+        does not keep them."""
         M, d = p.B * p.S, p.H * p.Dh
         res = x.reshape(M, d)
         if p.io_dtype != torch.float32:      # 16-bit input: widened once, fp32 inside
@@ -362,12 +365,12 @@ class FusedTransformer(BaselineTransformer):
                                        qkv=self._qkv_of(p, 0),
                                        want_residual=into_graph and len(self.layers) > 1)
             s, p.ops = p.entry(res)
-            p.res = res if s is None else s
-        else:
-            first = self.layers[0].norm1
-            p.res, p.h = K.add_mask_layernorm(res, None, p.keep, first.weight, first.bias,
-                                              first.eps, out_dtype=p.h_attn,
-                                              residual_dtype=p.rdtype, s_out=p.res, h_out=p.h)
+            return res if s is None else s
+        first = self.layers[0].norm1
+        s, p.h = K.add_mask_layernorm(res, None, p.keep, first.weight, first.bias, first.eps,
+                                      out_dtype=p.h_attn, residual_dtype=p.rdtype,
+                                      s_out=p.res, h_out=p.h)
+        return s
 
     def _layer_steps(self, p: "_Pass") -> None:
         """From the entry kernel's outputs to the last kernel's inputs."""
@@ -378,8 +381,8 @@ class FusedTransformer(BaselineTransformer):
         else:
             self._wide_steps(p)
 
-    def _leave(self, p: "_Pass") -> torch.Tensor:
-        """The last kernel of the stack, into a new tensor."""
+    def _leave(self, p: "_Pass", first: torch.Tensor) -> torch.Tensor:
+        """The last kernel of the stack, into a new tensor; `first`: what `_enter` returned."""
         norm = self.final_norm
         if p.narrow:
             if p.exit is None:
@@ -387,7 +390,7 @@ class FusedTransformer(BaselineTransformer):
                                           p.ctx, K.Planes) else p.ctx.device, p.keep, _norm_of(norm),
                                       tail=self._tail_of(p, len(self.layers) - 1),
                                       want_residual=False, out_dtype=p.io_dtype)
-            out = p.exit(p.res if len(self.layers) == 1 else p.last_res)[1]
+            out = p.exit(first if len(self.layers) == 1 else p.last_res)[1]
         else:
             out = K.add_mask_layernorm(p.last_res, p.f, p.keep, norm.weight, norm.bias, norm.eps,
                                        mask_out=True, out_dtype=p.io_dtype,
@@ -516,7 +519,7 @@ class _Pass:
     keep2d: Optional[torch.Tensor] = None   # [B, S] uint8
     kv_len: Optional[torch.Tensor] = None
     prefix: Optional[torch.Tensor] = None
-    res: Optional[torch.Tensor] = None      # residual rows after the entry kernel (or x itself)
+    res: Optional[torch.Tensor] = None      # residual rows after the entry kernel
     h: object = None                        # wide: its normalised rows
     ops: object = None                      # narrow: the first layer's q, k, v^T
     ctx: object = None                      # narrow: the last attention's output
@@ -557,16 +560,23 @@ class GraphRunner:
 
     The runner keeps no reference to its model (the model holds its runners): without the
     cycle a graph and its memory pool go when the model does, not at whatever later
-    allocation the cyclic garbage collector runs on."""
+    allocation the cyclic garbage collector runs on.
+
+    The graph's buffers are the runner's: a call holds the lock from the first write of them to
+    the launch of the last read, so threads that share a model and a stream each get the
+    forward of their own x. Calls on different streams are the caller's to order."""
 
     def __init__(self, model: FusedTransformer, x, mask):
+        self.lock = threading.Lock()
         with torch.inference_mode(False):
             # written by every call, from inference mode or not
             self.mask = None if mask is None else torch.empty(mask.shape, dtype=torch.bool,
                                                               device=mask.device)
         self._take_mask(mask)
         p = self.state = model._plan_pass(x, self.mask)
-        model._enter(p, x, into_graph=True)
+        first = model._enter(p, x, into_graph=True)
+        if len(model.layers) > 1 or not p.narrow:
+            p.res = first                      # a buffer that the captured kernels read
         self.graph, _ = _capture(lambda: model._eager_forward(x, self.mask),
                                  lambda: model._layer_steps(p))
 
@@ -578,14 +588,11 @@ class GraphRunner:
                 torch.ne(mask, 0, out=self.mask)
 
     def __call__(self, model, x, mask):
-        self._take_mask(mask)
-        p = self.state
-        model._enter(p, x, into_graph=True)
-        self.graph.replay()
-        out = model._leave(p)
-        if p.narrow:
-            p.res = None                       # it may be the caller's x
-        return out
+        with self.lock:
+            self._take_mask(mask)
+            first = model._enter(self.state, x, into_graph=True)
+            self.graph.replay()
+            return model._leave(self.state, first)
 
 
 class _BaselineGraph:
