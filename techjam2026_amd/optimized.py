@@ -345,7 +345,8 @@ class FusedTransformer(BaselineTransformer):
                      attn_name in K.P16_PRECISIONS, rs,
                      h_attn=K.planes_format(m_attn), ctx_fmt=K.planes_format(m_out),
                      h_ffn=K.planes_format(m_f1), hid_fmt=K.planes_format(m_f2),
-                     narrow=self._rows_fused(rdtype, modes), keep2d=keep2d)
+                     narrow=self._rows_fused(rdtype, modes), keep2d=keep2d,
+                     keep=None if keep2d is None else keep2d.reshape(B * S))
 
     def _enter(self, p: "_Pass", x: torch.Tensor, into_graph: bool = False) -> torch.Tensor:
         """The entry LayerNorm (narrow models: with the first q, k, v^T); returns the residual
@@ -469,6 +470,25 @@ class FusedTransformer(BaselineTransformer):
         p.last_res = res
 
     # --- graph path --------------------------------------------------------------
+    def _copies_pay(self, p: "_Pass") -> bool:
+        """Whether a call of this shape waits for the host, so that two small copies around a
+        graph of the whole stack cost less than launching its two ends beside the graph: those
+        launches take the host 55 us a call in narrow models and 70 in wide ones, a copy in and
+        a copy out 43 and 46, while on the device the copies add 6 to 10. The device's time is
+        estimated from its launches, the weights (each block of the row kernel streams all of
+        them) and the operations. Measured, ends / whole: one layer, d 32, 16 rows 53 / 41 us;
+        d 128, 4096 rows 55 / 43, 16384 rows 54 / 60; in separate kernels d 32, 16 rows
+        69 / 46, d 512, 256 rows 70 / 64, 1024 rows 73 / 79; four layers of d 128, 128 rows
+        80 / 86 and, in separate kernels, 122 / 126."""
+        cfg, layers = self.config, len(self.layers)
+        weights = sum(t.numel() * t.element_size() for w in self._layers_w for lin in w.values()
+                      for t in (lin.hi, lin.lo) if t is not None)
+        d = cfg.d_model
+        flops = p.B * p.S * layers * (8 * d * d + 4 * d * cfg.ffn_dim + 4 * p.S * d)
+        if p.narrow:
+            return 5.3 * (2 * layers + 2) + weights / 1e5 + flops / 1e8 < 42
+        return 2.8 * (7 * layers + 2) + weights / 1.2e6 + flops / 1e8 < 45
+
     def _graph_forward(self, x, valid_token_mask):
         key = (tuple(x.shape), x.dtype, x.device,
                None if valid_token_mask is None else
@@ -517,6 +537,7 @@ class _Pass:
     hid_fmt: object                         # GELU output -> ffn_out
     narrow: bool
     keep2d: Optional[torch.Tensor] = None   # [B, S] uint8
+    keep: Optional[torch.Tensor] = None     # the same as [B * S]
     kv_len: Optional[torch.Tensor] = None
     prefix: Optional[torch.Tensor] = None
     res: Optional[torch.Tensor] = None      # residual rows after the entry kernel
@@ -527,10 +548,6 @@ class _Pass:
     last_res: Optional[torch.Tensor] = None # residual rows before the last kernel
     entry: Optional[K.LayerBlock] = None    # narrow: the first and last row kernels
     exit: Optional[K.LayerBlock] = None
-
-    @property
-    def keep(self) -> Optional[torch.Tensor]:
-        return None if self.keep2d is None else self.keep2d.reshape(self.B * self.S)
 
 
 def _capture(warm, body):
@@ -555,8 +572,10 @@ class GraphRunner:
     Only the kernels between the first and the last are captured. The entry LayerNorm is
     launched on the caller's x and writes the graph's input buffers, the final one writes
     a new output tensor, so no call copies its input in or its output out (two passes over
-    the activation: 490 of 2710 us for 10000 x 128 rows of d 128, 0.8 of 49 ms at
-    4 x 65536 rows of d 1024), and a held result survives the next replay.
+    the activation: 490 of 2710 us for 10000 x 128 rows of d 128), and a held result survives
+    the next replay. Calls so short that the host's launches are their time
+    (`FusedTransformer._copies_pay`) capture the whole stack, between a copy of x and one of
+    the output.
 
     The runner keeps no reference to its model (the model holds its runners): without the
     cycle a graph and its memory pool go when the model does, not at whatever later
@@ -573,7 +592,18 @@ class GraphRunner:
             self.mask = None if mask is None else torch.empty(mask.shape, dtype=torch.bool,
                                                               device=mask.device)
         self._take_mask(mask)
+        self.x = None
         p = self.state = model._plan_pass(x, self.mask)
+        if model._copies_pay(p):
+            with torch.inference_mode(False):
+                self.x = torch.empty(x.shape, dtype=x.dtype, device=x.device)
+            self.x.copy_(x.detach())
+
+            def body():
+                return model._eager_forward(self.x, self.mask)
+
+            self.graph, self.out = _capture(body, body)
+            return
         first = model._enter(p, x, into_graph=True)
         if len(model.layers) > 1 or not p.narrow:
             p.res = first                      # a buffer that the captured kernels read
@@ -590,6 +620,10 @@ class GraphRunner:
     def __call__(self, model, x, mask):
         with self.lock:
             self._take_mask(mask)
+            if self.x is not None:
+                self.x.copy_(x.detach() if x.requires_grad else x)
+                self.graph.replay()
+                return self.out.clone()
             first = model._enter(self.state, x, into_graph=True)
             self.graph.replay()
             return model._leave(self.state, first)

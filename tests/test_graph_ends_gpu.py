@@ -8,11 +8,18 @@ import pytest
 import torch
 
 from techjam2026_amd.model import TransformerConfig
-from techjam2026_amd.optimized import LADDER, build_shared
+from techjam2026_amd.optimized import LADDER, FusedTransformer, build_shared
 from tests.test_stack_gpu import make_model
 
 pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda")
+
+
+@pytest.fixture(params=[False, True], ids=["ends", "whole"], autouse=True)
+def captured(request, monkeypatch):
+    """Both forms of the graph, whichever a shape would take: the kernels between the ends, and
+    the whole stack between two copies."""
+    monkeypatch.setattr(FusedTransformer, "_copies_pay", lambda self, p: request.param)
 
 
 @pytest.mark.parametrize("d,H,F,layers", [(128, 4, 192, 1), (64, 8, 64, 3), (512, 8, 512, 2)])

@@ -1,14 +1,16 @@
-"""The graph path's host side on the CPU: which inputs reach the entry kernels as they are, and
-that threads which share a runner keep their own data."""
+"""The graph path's host side on the CPU: which inputs reach the entry kernels as they are, that
+threads which share a runner keep their own data, and which calls capture the whole stack."""
 from __future__ import annotations
 
 import threading
 import time
+from types import SimpleNamespace
 
 import pytest
 import torch
 
-from techjam2026_amd.optimized import GraphRunner, _entry_rows
+from techjam2026_amd.model import TransformerConfig
+from techjam2026_amd.optimized import LADDER, FusedTransformer, GraphRunner, _entry_rows
 
 D, S = 32, 12
 
@@ -56,7 +58,8 @@ class _SlowGraph:
 
 def test_threads_that_share_a_runner_keep_their_own_rows():
     runner = GraphRunner.__new__(GraphRunner)            # no device: the captured part is a stand-in
-    runner.lock, runner.mask, runner.state, runner.graph = threading.Lock(), None, {}, _SlowGraph()
+    runner.lock, runner.x, runner.mask = threading.Lock(), None, None
+    runner.state, runner.graph = {}, _SlowGraph()
     wrong, model = [], _OneLayerModel()
 
     def calls(value):
@@ -72,3 +75,19 @@ def test_threads_that_share_a_runner_keep_their_own_rows():
     for t in threads:
         t.join(30)
     assert not wrong and not any(t.is_alive() for t in threads)
+
+
+@pytest.mark.parametrize("narrow,d,F,layers,B,S,whole", [
+    (True, 32, 32, 1, 1, 16, True), (False, 32, 32, 1, 1, 16, True),
+    (False, 128, 256, 1, 32, 128, True), (False, 512, 1024, 1, 2, 128, True),
+    (True, 128, 256, 1, 128, 128, False), (True, 128, 128, 4, 1, 128, False),
+    (False, 512, 1024, 1, 16, 128, False), (False, 512, 2048, 6, 16, 512, False),
+    (True, 64, 64, 1, 1, 4096, False),                   # attention over one long sequence
+])
+def test_calls_that_wait_for_the_host_capture_the_whole_stack(narrow, d, F, layers, B, S, whole):
+    model = FusedTransformer(TransformerConfig(B, S, d, max(1, d // 64), F, layers, True), LADDER["graph"])
+    plane = {"qkv": 3 * d * d, "out": d * d, "ffn_in": d * F, "ffn_out": d * F}
+    model._layers_w = [{k: SimpleNamespace(hi=torch.empty(n, dtype=torch.float16),
+                                           lo=torch.empty(n, dtype=torch.float16))
+                        for k, n in plane.items()} for _ in range(layers)]
+    assert model._copies_pay(SimpleNamespace(B=B, S=S, narrow=narrow)) == whole
