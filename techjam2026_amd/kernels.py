@@ -537,6 +537,41 @@ def layer_block_supported(d: int, ffn_dim: int, modes) -> bool:
     return d in LAYER_WIDTHS and ffn_dim % 32 == 0 and all(m in LAYER_MODES for m in modes)
 
 
+def _check_layer_operands(M: int, d: int, keep, norm, tail, qkv) -> None:
+    """The kernel reads its operands at the extents that M, d and the feed-forward width give:
+    what does not have them is refused here."""
+    assert tail is not None or qkv is not None, "layer_block: neither a tail nor a projection"
+    row, act = (d,), (M, d)
+    dense = [(norm[0], row, torch.float32), (norm[1], row, torch.float32)]
+    linears = []
+    if keep is not None:
+        dense.append((keep, (M,), torch.uint8))
+    if tail is not None:
+        ctx, out, norm2, f1, f2 = tail
+        dense += (norm2[0], row, torch.float32), (norm2[1], row, torch.float32)
+        if isinstance(ctx, Planes):
+            dense += (ctx.hi, act, torch.float16), (ctx.lo, act, torch.float16)
+        else:
+            assert out.mode != L.MMA_F16X3, "layer_block: an f16x3 out_proj reads ctx planes"
+            dense.append((ctx, act, torch.float16))
+        linears = [(out, d, d), (f1, f1.N, d), (f2, d, f1.N)]
+    if qkv is not None:
+        w, B, S, H, Dh, single = qkv
+        linears.append((w, 3 * d, d))
+        assert B * S == M and H * Dh == d, f"layer_block: {B} x {S} tokens of {H} x {Dh} for {act}"
+        assert not single or w.mode == L.MMA_F16X3, "single-plane k / v^T from an f16x3 projection"
+    device = norm[0].device
+    for t, shape, dtype in dense:
+        assert t.shape == shape and t.dtype == dtype and t.is_contiguous() and t.device == device, \
+            f"layer_block: {tuple(t.shape)} {t.dtype} on {t.device}, needs a dense {shape} {dtype}"
+    for w, N, k in linears:
+        assert w.N == N and w.K == k and w.mode in LAYER_MODES and w.hi.device == device, \
+            f"layer_block: weight [{w.N}, {w.K}] in mode {w.mode}, needs [{N}, {k}]"
+        assert w.bias is not None and w.bias.shape == (N,), "layer_block: a linear's bias"
+    if device.type != "cuda":
+        raise RuntimeError("libkf950 kernels need device tensors")
+
+
 class LayerBlock:
     """The row-wise part of a layer as one launch (kf_layer_block), prepared: everything but
     the residual rows and the output is fixed, so a call sets two pointers and launches.
@@ -548,12 +583,15 @@ class LayerBlock:
     A call takes res [M, d] (fp32, unit column stride, 16-byte aligned rows) and returns
     (s or None, AttnOperands) with `qkv`, else (s or None, y [M, d] in `out_dtype`); s and the
     operands are buffers of this object, written again by each call, y is a new tensor.
-    `rows` forces the rows per block (16 / 32 / 64; 0: automatic; same results)."""
+    `rows` forces the rows per block (16 / 32 / 64; 0: automatic; same results). `check` False:
+    the caller has made sure that the operands fit (8 us a block)."""
 
     def __init__(self, M: int, d: int, device, keep: Optional[torch.Tensor], norm, tail=None,
                  qkv=None, want_residual: bool = True, out_dtype: torch.dtype = torch.float32,
-                 rows: int = 0):
-        _need_cuda(keep)
+                 rows: int = 0, check: bool = True):
+        if check:
+            _check_layer_operands(M, d, keep, norm, tail, qkv)
+        self.device = norm[0].device
         self.s = torch.empty((M, d), dtype=torch.float32, device=device) if want_residual else None
         self.ops = None
         self.out_dtype = out_dtype
@@ -591,7 +629,7 @@ class LayerBlock:
     def __call__(self, res: torch.Tensor):
         # a copy: another thread's call can't change the pointers between here and the launch
         a = L.LayerArgs.from_buffer_copy(self.args)
-        assert res.is_cuda and res.dtype == torch.float32 and tuple(res.shape) == (a.M, a.d) \
+        assert res.device == self.device and res.dtype == torch.float32 and tuple(res.shape) == (a.M, a.d) \
             and res.stride(1) == 1
         a.res, a.ld_res = res.data_ptr(), res.stride(0)
         result = self.ops

@@ -364,7 +364,8 @@ class FusedTransformer(BaselineTransformer):
                 # reads it), unless a captured layer reads it
                 p.entry = K.LayerBlock(M, d, x.device, p.keep, _norm_of(self.layers[0].norm1),
                                        qkv=self._qkv_of(p, 0),
-                                       want_residual=into_graph and len(self.layers) > 1)
+                                       want_residual=into_graph and len(self.layers) > 1,
+                                       check=False)
             s, p.ops = p.entry(res)
             return res if s is None else s
         first = self.layers[0].norm1
@@ -390,7 +391,7 @@ class FusedTransformer(BaselineTransformer):
                 p.exit = K.LayerBlock(p.B * p.S, p.H * p.Dh, p.ctx.hi.device if isinstance(
                                           p.ctx, K.Planes) else p.ctx.device, p.keep, _norm_of(norm),
                                       tail=self._tail_of(p, len(self.layers) - 1),
-                                      want_residual=False, out_dtype=p.io_dtype)
+                                      want_residual=False, out_dtype=p.io_dtype, check=False)
             out = p.exit(first if len(self.layers) == 1 else p.last_res)[1]
         else:
             out = K.add_mask_layernorm(p.last_res, p.f, p.keep, norm.weight, norm.bias, norm.eps,
@@ -441,14 +442,22 @@ class FusedTransformer(BaselineTransformer):
     # --- narrow models: one kernel per layer beside attention ----------------------
     def _rows_fused(self, rdtype, modes) -> bool:
         """Whether the row-wise part of each layer runs as one kernel (kf_layer_block): a
-        width it serves, fp16-family stages and fp32 norm parameters (16-bit models keep
-        theirs in 16 bits) that it can read in 16-byte pieces."""
-        cfg = self.config
+        width it serves, fp16-family stages, weights of the shapes it reads and fp32 norm
+        parameters (16-bit models keep theirs in 16 bits) that it can read in 16-byte pieces."""
+        d = self.config.d_model
+
+        def fits(w):
+            qkv, out, f1, f2 = w["qkv"], w["out"], w["ffn_in"], w["ffn_out"]
+            return (K.layer_block_supported(d, f1.N, modes)
+                    and (qkv.N, qkv.K, out.N, out.K, f1.K, f2.N, f2.K) == (3 * d, d, d, d, d, d, f1.N)
+                    and all(lin.bias is not None and lin.bias.shape == (lin.N,)
+                            for lin in (qkv, out, f1, f2)))
+
         norms = [n for layer in self.layers for n in (layer.norm1, layer.norm2)] + [self.final_norm]
         return (rdtype == torch.float32
-                and K.layer_block_supported(cfg.d_model, cfg.ffn_dim, modes)
-                and all(t.dtype == torch.float32 and t.is_contiguous() and t.data_ptr() % 16 == 0
-                        for n in norms for t in (n.weight, n.bias)))
+                and all(fits(w) for w in self._layers_w)
+                and all(t.dtype == torch.float32 and t.shape == (d,) and t.is_contiguous()
+                        and t.data_ptr() % 16 == 0 for n in norms for t in (n.weight, n.bias)))
 
     def _qkv_of(self, p: "_Pass", i: int):
         return self._layers_w[i]["qkv"], p.B, p.S, p.H, p.Dh, p.single_attn
@@ -466,7 +475,8 @@ class FusedTransformer(BaselineTransformer):
             p.ctx = self._attend(p, ops)
             if i + 1 < len(self.layers):
                 res, ops = K.layer_block(res, p.keep, _norm_of(self.layers[i + 1].norm1),
-                                         tail=self._tail_of(p, i), qkv=self._qkv_of(p, i + 1))
+                                         tail=self._tail_of(p, i), qkv=self._qkv_of(p, i + 1),
+                                         check=False)
         p.last_res = res
 
     # --- graph path --------------------------------------------------------------
