@@ -440,10 +440,22 @@ class FusedTransformer(BaselineTransformer):
         p.last_res, p.f = res, f
 
     # --- narrow models: one kernel per layer beside attention ----------------------
+    # The most weight bytes of a layer that the row kernel takes. Each of its blocks streams all
+    # of them at about 100 GB/s, the chain of a launch however few the rows, where separate
+    # kernels spread them over the chip. Six layers, f16x3, row kernel / today's separate
+    # kernels / separate kernels with 128 x 128 GEMM tiles, us: d 128, F 512 (0.8 MB), 256 rows
+    # 124 / 190 / 312; d 256, F 1024 (3.1 MB), 256 rows 272 / 212 / 430, 4096 rows 350 / 456 / 535,
+    # 16384 rows 862 / 1045 / 1103; d 256, F 4096 (9.4 MB), 64 rows 664 / 264 / 682, 4096 rows
+    # 737 / 776 / 993; F 8192 (17.8 MB), 64 rows 1177 / 355 / 1065. The line lies where the row
+    # kernel would lose to what it replaced. With few rows the separate kernels win earlier
+    # (from 2 MB at 256 rows), but a rule on rows would give a sequence other last bits in
+    # another batch.
+    ROW_KERNEL_BYTES = 8 << 20
+
     def _rows_fused(self, rdtype, modes) -> bool:
         """Whether the row-wise part of each layer runs as one kernel (kf_layer_block): a
-        width it serves, fp16-family stages, weights of the shapes it reads and fp32 norm
-        parameters (16-bit models keep theirs in 16 bits) that it can read in 16-byte pieces."""
+        width it serves, fp16-family stages, weights of the shapes it reads, not too many of
+        them for one block to stream, and fp32 norm parameters (16-bit models keep theirs in 16 bits) that it can read in 16-byte pieces."""
         d = self.config.d_model
 
         def fits(w):
@@ -456,6 +468,7 @@ class FusedTransformer(BaselineTransformer):
         norms = [n for layer in self.layers for n in (layer.norm1, layer.norm2)] + [self.final_norm]
         return (rdtype == torch.float32
                 and all(fits(w) for w in self._layers_w)
+                and max(self._layer_weight_bytes()) <= self.ROW_KERNEL_BYTES
                 and all(t.dtype == torch.float32 and t.shape == (d,) and t.is_contiguous()
                         and t.data_ptr() % 16 == 0 for n in norms for t in (n.weight, n.bias)))
 
@@ -480,6 +493,10 @@ class FusedTransformer(BaselineTransformer):
         p.last_res = res
 
     # --- graph path --------------------------------------------------------------
+    def _layer_weight_bytes(self) -> List[int]:
+        return [sum(t.numel() * t.element_size() for lin in w.values() for t in (lin.hi, lin.lo)
+                    if t is not None) for w in self._layers_w]
+
     def _copies_pay(self, p: "_Pass") -> bool:
         """Whether a call of this shape waits for the host, so that two small copies around a
         graph of the whole stack cost less than launching its two ends beside the graph: those
@@ -491,8 +508,7 @@ class FusedTransformer(BaselineTransformer):
         69 / 46, d 512, 256 rows 70 / 64, 1024 rows 73 / 79; four layers of d 128, 128 rows
         80 / 86 and, in separate kernels, 122 / 126."""
         cfg, layers = self.config, len(self.layers)
-        weights = sum(t.numel() * t.element_size() for w in self._layers_w for lin in w.values()
-                      for t in (lin.hi, lin.lo) if t is not None)
+        weights = sum(self._layer_weight_bytes())
         d = cfg.d_model
         flops = p.B * p.S * layers * (8 * d * d + 4 * d * cfg.ffn_dim + 4 * p.S * d)
         if p.narrow:

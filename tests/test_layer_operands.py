@@ -79,3 +79,19 @@ def test_a_model_whose_weights_do_not_fit_keeps_the_separate_kernels():
     assert not fused(ffn_out=_linear(D, F - 32))
     assert not fused(out=_linear(D, D, bias=False))
     assert not fused(modes=(L.MMA_BF16X3,) * 4)
+
+
+@pytest.mark.parametrize("d,ffn,planes,row_kernel", [
+    (256, 1024, 2, True), (256, 3072, 2, True), (256, 4096, 2, False), (256, 8192, 1, False),
+    (256, 6144, 1, True), (128, 4096, 2, True), (32, 4096, 2, True)])
+def test_layers_of_many_weights_keep_the_separate_kernels(d, ffn, planes, row_kernel):
+    mode = L.MMA_F16X3 if planes == 2 else L.MMA_F16
+
+    def lin(n, k):
+        w = _linear(n, k, mode)
+        w.lo = w.hi if planes == 2 else None
+        return w
+
+    model = FusedTransformer(TransformerConfig(1, 64, d, 1, 32, 1, True), LADDER["graph"])
+    model._layers_w = [dict(qkv=lin(3 * d, d), out=lin(d, d), ffn_in=lin(ffn, d), ffn_out=lin(d, ffn))]
+    assert model._rows_fused(torch.float32, (mode,) * 4) == row_kernel
