@@ -138,6 +138,12 @@ int kf_gemm_tiled(const void* a, const void* a_lo, int a_dtype, int64_t lda,
  * BM, BN, BK, LDS stages, wavefronts per block, 1 for the LDS-DMA kernel. Host only. */
 int kf_gemm_tile_info(int tile, int* info);
 
+/* Host-only check hook (no reference counterpart; launches nothing): the tile id that `tile` 0
+ * stands for in a product with 16-bit A, K % 32 == 0 (`epilogue` 0: plain, 1: GELU, 2: the
+ * attention layout of kf_gemm_qkv) on a device of `cus` compute units; -1 for bad arguments.
+ * For CPU tests of the choice against measured times. */
+int kf_gemm_tile_choice(int64_t M, int64_t N, int64_t K, int mode, int epilogue, int cus);
+
 /* Per-sequence key extent of a [B, S] validity mask: kv_len[b] = 1 + the last valid
  * position (0 if none), prefix[b] = 1 when positions [0, kv_len[b]) are all valid.
  * Prepares kf_flash_fwd's skip of fully padded key/query blocks (the reference applies

@@ -28,7 +28,7 @@ EXPORTS = ("kf_abi_version", "kf_last_error", "kf_device_ok", "kf_add_mask_ln", 
            "kf_gemm", "kf_gemm_tiled", "kf_gemm_tile_info", "kf_mask_prep", "kf_gemm_qkv",
            "kf_gemm_qkv_tiled", "kf_attn_prep", "kf_flash_tile_info", "kf_flash_block_map",
            "kf_flash_fwd", "kf_flash_attention_static", "kf_layer_block",
-           "kf_fragments")
+           "kf_fragments", "kf_gemm_tile_choice")
 
 
 class KernelError(RuntimeError):
@@ -93,6 +93,8 @@ def _declare(h: ctypes.CDLL) -> None:
                                 c_int, c_i64, c_i64, c_i64, c_i64, c_int, c_int, c_int, c_vp]
     h.kf_gemm_tile_info.restype = c_int
     h.kf_gemm_tile_info.argtypes = [c_int, c_vp]
+    h.kf_gemm_tile_choice.restype = c_int
+    h.kf_gemm_tile_choice.argtypes = [c_i64, c_i64, c_i64, c_int, c_int, c_int]
     h.kf_flash_block_map.restype = c_int
     h.kf_flash_block_map.argtypes = [c_int, c_int, c_int, c_int, c_vp]
     h.kf_mask_prep.restype = c_int

@@ -23,22 +23,23 @@ __global__ void split_kernel(const float* src, int64_t n, E* hi, E* lo) {
 // epilogue's weight (plain, GELU, QKV). q is what a whole-chip rule cannot see: tiles of
 // 128 x 128 for 3001 x 768 outputs leave 112 of 256 CUs idle, 256 x 256 ones for 8192 x 3072
 // run a second round half empty. Two blocks sharing a CU take about twice as long as one, so
-// residency does not enter. a, e and s are fitted per operand planes to every tile timed over 60
-// to 64 products (M 64 ... 70000, N and K 256 ... 4096, three epilogues); over those products
-// the choice is within 1-2 % of the fastest tile (geometric mean), 20-25 % faster than a
-// fixed preference for 128 x 128 and, on large grids, 256 x 256 tiles, and never more than
-// 11 % slower than it. Measured, before -> after: f16x3 256 x 512 x 2048 35.8 -> 9.8 us,
-// 1024 x 768 x 3072 59 -> 24; fp16 3001 x 768 x 3072 34.7 -> 30.7, 8192 x 4096 x 1024
-// 101 -> 75; f16x2 8192 x 768 x 3072 92 -> 72.
+// residency does not enter. a, e and s were fitted per operand planes; profiles/gemm_tile_times.txt
+// holds 573 products (M 16 ... 100000, N 32 ... 12288, K 128 ... 16384) timed with every tile, to
+// check or redo the fit. There the choice takes 1.02 times the fastest tile's time (geometric
+// mean) and a fixed preference for 128 x 128 and, on large grids, 256 x 256 tiles 1.39 times; in
+// 14 of the 573 the choice is more than 4 % behind that preference, by up to 10 %. Measured,
+// preference -> choice: f16x3 256 x 512 x 2048 35.8 -> 9.8 us, 1024 x 768 x 3072 59 -> 24;
+// fp16 3001 x 768 x 3072 34.7 -> 30.7, 8192 x 4096 x 1024 101 -> 75; f16x2 8192 x 768 x 3072
+// 92 -> 72.
 struct TileCost { int tile; float a, e; };
 struct ModeCost { float s[3]; TileCost tiles[11]; int n; };
 static const ModeCost kCostSplit = {{1.0f, 1.8f, 1.5f},
     {{DMA_256x256k32s2w8, 65.f, 7.9f}, {DMA_128x256k32s3w8, 37.f, 4.4f},
-     {DMA_128x128k64s2w8, 20.f, 1.9f}, {DMA_128x64k64s3w8, 13.f, 1.0f},
+     {DMA_128x128k64s2w8, 20.6f, 1.9f}, {DMA_128x64k64s3w8, 13.f, 1.0f},
      {DMA_64x64k64s4w4, 9.2f, 0.85f}, {DMA_32x64k128s3w4, 6.0f, 0.62f},
      {DMA_32x32k128s3w4, 3.9f, 0.29f}, {DMA_128x128k32s3w8, 22.f, 2.1f},
      {DMA_64x64k32s3w4, 10.f, 0.3f}}, 9};
-static const ModeCost kCostSingle = {{1.0f, 1.4f, 1.2f},
+static const ModeCost kCostSingle = {{1.0f, 1.4f, 1.5f},
     {{DMA_256x256k64s2w8, 22.f, 9.5f}, {DMA_128x256k64s3w8, 13.f, 4.7f},
      {DMA_128x128k64s2w8, 8.4f, 1.3f}, {DMA_128x64k64s3w8, 5.4f, 0.72f},
      {DMA_64x64k64s4w4, 3.5f, 0.34f}, {DMA_32x64k128s3w4, 2.4f, 0.28f},
@@ -53,11 +54,10 @@ static const ModeCost kCostF16x2 = {{1.0f, 1.4f, 1.6f},
      {DMA_128x128k32s3w8, 15.f, 2.1f}, {DMA_64x64k32s3w4, 8.5f, 0.3f}}, 10};
 enum { EPI_PLAIN = 0, EPI_GELU = 1, EPI_QKV = 2 };
 
-static int pick_dma(int64_t M, int64_t N, int64_t K, int mode, int epilogue) {
+static int pick_dma(int64_t M, int64_t N, int64_t K, int mode, int epilogue, int64_t cus) {
   if (K < 128) return epilogue == EPI_QKV ? DMA_128x64k32s3w4 : DMA_64x64k32s3w4;
   const ModeCost& mc = mode == KF_MMA_F16X3 || mode == KF_MMA_BF16X3 ? kCostSplit
                      : mode == KF_MMA_F16X2 ? kCostF16x2 : kCostSingle;
-  const int64_t cus = cu_count();
   int best = DMA_128x128k32s4w8;
   float least = 3.4e38f;
   for (int i = 0; i < mc.n; ++i) {
@@ -67,7 +67,15 @@ static int pick_dma(int64_t M, int64_t N, int64_t K, int mode, int epilogue) {
     // four stages hide the memory latency of a lone block over a long K (fp16 3001 x 768 x
     // 3072: 34.9 -> 29.7 us), but they leave no room for a second one
     if (mc.tiles[i].tile == DMA_128x128k64s4w8 && tiles > cus) continue;
-    const float cost = (float)((tiles + cus - 1) / cus) *
+    const int64_t q = (tiles + cus - 1) / cus;
+    // The split modes' 128 x 256 tile copies 64-byte halves of a row's 128-byte lines, k-step by
+    // k-step. Over a long K and several rounds, or with more weights than the caches keep, the
+    // other halves are fetched again: f16x3 8329 x 6528 x 3072 979 us against 828 with 256 x 256,
+    // 553 x 12288 x 4096 248 against 185 with 128 x 128 x 64. Up to three rounds it is the best by
+    // 3 to 20 % (2197 x 9216 x 3072 390 against 419 and 423).
+    if (&mc == &kCostSplit && mc.tiles[i].tile == DMA_128x256k32s3w8 && K >= 3072 &&
+        (q > 3 || 4 * N * K > 170000000)) continue;
+    const float cost = (float)q *
                        (mc.tiles[i].a * (float)K * (1.0f / 1024.0f) + mc.tiles[i].e * mc.s[epilogue]);
     if (cost < least) { least = cost; best = mc.tiles[i].tile; }
   }
@@ -81,7 +89,7 @@ static int pick_tile(int requested, int64_t M, int64_t N, int64_t K, bool a16, i
   int t = requested;
   if (t >= DMA_FIRST && (!a16 || K % kTileInfo[t].bk)) t = TILE_AUTO;
   if (mode == KF_MMA_F16X2 && t != TILE_AUTO && t < DMA_FIRST) t = TILE_AUTO;
-  if (t == TILE_AUTO && a16 && K % 32 == 0) t = pick_dma(M, N, K, mode, epilogue);
+  if (t == TILE_AUTO && a16 && K % 32 == 0) t = pick_dma(M, N, K, mode, epilogue, cu_count());
   if (t == TILE_AUTO) {
     const int64_t blocks128 = ((M + 127) / 128) * ((N + 127) / 128);
     if (blocks128 >= 512) t = TILE_128x128k32;
@@ -116,6 +124,15 @@ extern "C" int kf_gemm_tile_info(int tile, int* info) {
   info[0] = t.bm; info[1] = t.bn; info[2] = t.bk; info[3] = t.stages; info[4] = t.waves;
   info[5] = t.dma;
   return KF_OK;
+}
+
+// Check hook (declared in kf950.h; host only, launches nothing): the tile that a call without
+// one runs, for 16-bit A on a device of `cus` compute units.
+extern "C" int kf_gemm_tile_choice(int64_t M, int64_t N, int64_t K, int mode, int epilogue, int cus) {
+  if (M < 1 || N < 1 || K < 32 || K % 32 || M > (1LL << 30) || N > (1LL << 30) || K > (1LL << 30) ||
+      mode < KF_MMA_F16 || mode > KF_MMA_F16X2 || epilogue < EPI_PLAIN || epilogue > EPI_QKV || cus < 1)
+    return -1;
+  return pick_dma(M, N, K, mode, epilogue, cus);
 }
 
 extern "C" int kf_gemm_tiled(const void* a, const void* a_lo, int a_dtype, int64_t lda,
