@@ -817,13 +817,13 @@ template <int MODE, int HDP> constexpr bool flash_serves_all() {
   return !(HDP == 128 && ModeTraits<MODE>::split);
 }
 
-template <int MODE, int QT, int HDP, int VAR = kVarNone, bool SMALL = false>
+template <int MODE, int QT, int HDP, int VAR, bool SMALL, bool GEN>
 __global__ __launch_bounds__((FlashTile<HDP, ModeTraits<MODE>::split ? 2 : 1, SMALL>::NTH))
 __attribute__((amdgpu_waves_per_eu(flash_waves_per_simd<MODE, HDP, VAR>())))
 void flash_fwd_kernel(FlashArgs a) {
   __shared__ __attribute__((aligned(1024)))
   typename ModeTraits<MODE>::elem smem[flash_stage_elems<MODE, HDP>()];
-  flash_fwd_block<MODE, QT, HDP, VAR, flash_serves_all<MODE, HDP>(), SMALL>(a, blockIdx.x, gridDim.x, smem);
+  flash_fwd_block<MODE, QT, HDP, VAR, GEN, SMALL>(a, blockIdx.x, gridDim.x, smem);
 }
 
 // The rows whose mask is no prefix, beside a kernel that serves the prefix ones (head_dim 8
@@ -2321,17 +2321,26 @@ static void launch_fwd(const FlashArgs& a, hipStream_t st) {
   // all of them run at once; head_dim 64 and 256 have one group a wavefront already. Same
   // results: a row takes the same steps in the same order.
   const bool prefix_rows = all || a.keep == nullptr || (a.kv_len && a.prefix);
+  // calls without a mask run an instantiation without the code of general rows, which costs 3 to
+  // 6 % (8 heads of 4096 keys of 64, f16x3, causal: 96.2 against 102.3 us; 96 of 1024 keys of 8,
+  // fp16: 24.9 against 27.0)
+  const bool masked = a.keep != nullptr;
   if constexpr (HDP == 32 || (HDP == 128 && ModeTraits<MODE>::split)) {
     if (prefix_rows && blocks * (HDP == 128 ? 2 : 1) <= cu_count()) {
       using FS = FlashTile<HDP, ModeTraits<MODE>::split ? 2 : 1, true>;
       const int64_t small = (int64_t)((a.S + FS::BM - 1) / FS::BM) * a.B * a.H;
-      hipLaunchKernelGGL((flash_fwd_kernel<MODE, QT, HDP, VAR, true>), dim3((unsigned)small), dim3(FS::NTH), 0, st, a);
+      if (masked)
+        hipLaunchKernelGGL((flash_fwd_kernel<MODE, QT, HDP, VAR, true, all>), dim3((unsigned)small), dim3(FS::NTH), 0, st, a);
+      else
+        hipLaunchKernelGGL((flash_fwd_kernel<MODE, QT, HDP, VAR, true, false>), dim3((unsigned)small), dim3(FS::NTH), 0, st, a);
       if constexpr (!all) launch_general<MODE, QT, HDP, VAR>(a, st);
       return;
     }
   }
-  if (prefix_rows)
-    hipLaunchKernelGGL((flash_fwd_kernel<MODE, QT, HDP, VAR>), dim3((unsigned)blocks), dim3(FT::NTH), 0, st, a);
+  if (prefix_rows && masked)
+    hipLaunchKernelGGL((flash_fwd_kernel<MODE, QT, HDP, VAR, false, all>), dim3((unsigned)blocks), dim3(FT::NTH), 0, st, a);
+  else if (prefix_rows)
+    hipLaunchKernelGGL((flash_fwd_kernel<MODE, QT, HDP, VAR, false, false>), dim3((unsigned)blocks), dim3(FT::NTH), 0, st, a);
   if constexpr (!all) launch_general<MODE, QT, HDP, VAR>(a, st);
 }
 

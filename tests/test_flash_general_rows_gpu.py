@@ -47,3 +47,20 @@ def test_mixed_masks_match_float64(mode, hd, B, H, S, causal):
     assert err < TOL[mode], f"off by {err:.2e}"
     dead = ~(s > -float("inf")).any(-1)
     assert torch.count_nonzero(got[dead]) == 0
+
+
+@pytest.mark.parametrize("mode", [L.MMA_F16, L.MMA_F16X3, L.MMA_BF16X3])
+@pytest.mark.parametrize("hd", [8, 16, 32, 64, 128, 256])
+@pytest.mark.parametrize("B,H,S", [(1, 1, 1), (2, 3, 65), (2, 2, 333), (40, 8, 130)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_no_mask_equals_a_mask_of_ones(mode, hd, B, H, S, causal):
+    """Calls without a mask run instantiations without the mask code: the same bits."""
+    g = torch.Generator(device=DEV).manual_seed(hd + S)
+    dt = torch.float16 if mode == L.MMA_F16 else torch.float32
+    q, k, v = (torch.randn(B, H, S, hd, device=DEV, generator=g).to(dt) for _ in range(3))
+    ones = torch.ones(B, S, dtype=torch.bool, device=DEV)
+    want = K.flash_attention(q, k, v, keep=ones, causal=causal, mode=mode)
+    got = K.flash_attention(q, k, v, causal=causal, mode=mode)
+    assert torch.equal(got, want)
+    p16 = [K.flash_attention(q, k, v, keep=m, causal=causal, mode=mode, p16=True) for m in (None, ones)]
+    assert torch.equal(*p16)
