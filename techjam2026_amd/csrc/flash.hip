@@ -50,8 +50,8 @@ __global__ __launch_bounds__(256) void mask_prep_kernel(const void* keep, int dt
 // [.., hd, keys], zero in the pad columns [S, roundup(S, 8)). HBM-bound: a thread takes an
 // 8 x 8 block (eight keys, one 8-element chunk of d) of v and turns it in registers, or the
 // same block of k. A wavefront's 64 blocks are CW chunks (whole 128-byte pieces of 16-bit rows
-// from head_dim 64) by 64 / CW key blocks, so V^T leaves in 16-byte stores that fill whole
-// lines too. One thread per key and chunk, storing its eight columns of V^T in 2-byte
+// from head_dim 64) by 64 / CW key blocks (kf_attn_prep: of one head or of several), so V^T
+// leaves in 16-byte stores that fill whole lines too. One thread per key and chunk, storing its eight columns of V^T in 2-byte
 // pieces, took 65 of 1131 us of fp16 attention over 2 x 16 heads of 16384 keys (1095 now) and
 // 29.6 of 104.6 us of fp32 attention over 4 x 8 heads of 1001 keys of 128 (87.0 now).
 struct PrepArgs {
@@ -61,24 +61,21 @@ struct PrepArgs {
   void* vt_hi; void* vt_lo; int64_t ts0, ts1, ts2;
   int B, H, S, hd;
   int vec_k, vec_v;        // 16-byte aligned outputs (base and strides)
+  uint32_t per;            // key blocks that a (b, h) takes of the wavefronts' lanes
 };
 
 template <int IT, typename E, bool TWO>
 __global__ __launch_bounds__(256) void attn_prep_kernel(PrepArgs a) {
   typedef E V8 __attribute__((ext_vector_type(8)));
   const bool is_v = blockIdx.y == 0;
-  const int cpr = a.hd / 8, cw = cpr < 8 ? cpr : 8;
-  const int nsb = (a.S + 7) / 8;                     // key blocks per (b, h)
-  const int sw = 64 / cw, spans = (nsb + sw - 1) / sw, groups = cpr / cw;
-  const int lane = threadIdx.x & 63;
-  int64_t w = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (w >= (int64_t)a.B * a.H * spans * groups) return;
-  const int c = (int)(w % groups) * cw + lane % cw;
-  w /= groups;
-  const int sb = (int)(w % spans) * sw + lane / cw;
-  w /= spans;
-  const int h = (int)(w % a.H), b = (int)(w / a.H);
-  if (sb >= nsb) return;
+  const uint32_t cpr = a.hd / 8, cw = cpr < 8 ? cpr : 8, groups = cpr / cw;   // powers of two
+  const uint32_t lane = threadIdx.x & 63;
+  const uint32_t w = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);     // wavefront
+  const int c = (int)((w % groups) * cw + lane % cw);
+  const uint32_t block = (w / groups) * (64 / cw) + lane / cw;                // key block of all
+  const uint32_t sb = block % a.per, bh = block / a.per;
+  if (bh >= (uint32_t)a.B * a.H || 8 * sb >= (uint32_t)a.S) return;
+  const int h = (int)(bh % a.H), b = (int)(bh / a.H);
   const int s0 = 8 * sb, d = 8 * c;
   const void* src = is_v ? a.v : a.k;
   const int64_t at = is_v ? b * a.vs0 + h * a.vs1 + d : b * a.ks0 + h * a.ks1 + d;
@@ -241,21 +238,34 @@ extern "C" int kf_attn_prep(const void* k, const int64_t* ks, const void* v, con
   static const int64_t zero4[4] = {0, 0, 0, 1};
   const int64_t* kst = with_k ? ks : zero4;
   const int64_t* kost = with_k ? kos : zero4;
-  const int64_t cpr = hd / 8, cw = cpr < 8 ? cpr : 8, sw = 64 / cw;
-  const int64_t waves = B * H * (((S + 7) / 8 + sw - 1) / sw) * (cpr / cw);
-  if ((waves + 3) / 4 > 0x7fffffffLL) { kf_set_error("kf_attn_prep: problem too large"); return KF_EUNSUPPORTED; }
-  const dim3 grid((unsigned)((waves + 3) / 4), with_k ? 2 : 1);
+  // A wavefront takes sw key blocks. A (b, h) starts a wavefront of its own where that leaves
+  // under half of the lanes idle (its V^T lines are then written by one wavefront: 2048 heads of
+  // 33 keys of 256, fp32, 57 against 65 us); shorter ones share wavefronts (65536 heads of 4 keys
+  // of 8, fp32, 120 -> 14 us). Few wavefronts go one to a block, over more CUs (8 heads of 4096
+  // keys of 8, fp32, 6.8 -> 4.4 us); more of them four to a block, since the heads of a token share
+  // lines and so an XCD's L2 (512 heads of 512 keys of 8, fp16, 11.2 -> 6.6 us).
+  const int64_t cpr = hd / 8, cw = cpr < 8 ? cpr : 8, sw = 64 / cw, nsb = (S + 7) / 8;
+  const int64_t per = 2 * nsb >= sw ? (nsb + sw - 1) / sw * sw : nsb;
+  // key blocks and wavefronts are counted in 32 bits (2^31 of them write at least 128 GB)
+  if (B > 0x7fffffffLL || H > 0x7fffffffLL || per > 0x7fffffffLL || B * H > 0x7fffffffLL / per) {
+    kf_set_error("kf_attn_prep: problem too large");
+    return KF_EUNSUPPORTED;
+  }
+  const int64_t waves = (B * H * per + sw - 1) / sw * (cpr / cw);
+  if (waves > 0x7fffffffLL) { kf_set_error("kf_attn_prep: problem too large"); return KF_EUNSUPPORTED; }
+  const int wpb = waves <= cu_count() ? 1 : 4;               // wavefronts a block
+  const dim3 grid((unsigned)((waves + wpb - 1) / wpb), with_k ? 2 : 1);
   hipStream_t st = (hipStream_t)stream;
   const PrepArgs pa{k, kst[0], kst[1], kst[2], v, vs[0], vs[1], vs[2], k_hi, k_lo, kost[0], kost[1],
                     kost[2], vt_hi, vt_lo, vts[0], vts[1], vts[2], (int)B, (int)H, (int)S, (int)hd,
                     with_k && al16s(k_hi, split ? k_lo : nullptr, kos),
-                    al16s(vt_hi, split ? vt_lo : nullptr, vts)};
+                    al16s(vt_hi, split ? vt_lo : nullptr, vts), (uint32_t)per};
   const bool bf = mode == KF_MMA_BF16 || mode == KF_MMA_BF16X3;
 #define KF_PREP(IT)                                                                                  \
-  if (bf && split) hipLaunchKernelGGL((attn_prep_kernel<IT, __bf16, true>), grid, dim3(256), 0, st, pa);  \
-  else if (bf) hipLaunchKernelGGL((attn_prep_kernel<IT, __bf16, false>), grid, dim3(256), 0, st, pa);     \
-  else if (split) hipLaunchKernelGGL((attn_prep_kernel<IT, _Float16, true>), grid, dim3(256), 0, st, pa); \
-  else hipLaunchKernelGGL((attn_prep_kernel<IT, _Float16, false>), grid, dim3(256), 0, st, pa)
+  if (bf && split) hipLaunchKernelGGL((attn_prep_kernel<IT, __bf16, true>), grid, dim3(64 * wpb), 0, st, pa);  \
+  else if (bf) hipLaunchKernelGGL((attn_prep_kernel<IT, __bf16, false>), grid, dim3(64 * wpb), 0, st, pa);     \
+  else if (split) hipLaunchKernelGGL((attn_prep_kernel<IT, _Float16, true>), grid, dim3(64 * wpb), 0, st, pa); \
+  else hipLaunchKernelGGL((attn_prep_kernel<IT, _Float16, false>), grid, dim3(64 * wpb), 0, st, pa)
   switch (in_dtype) {
     case KF_F32: KF_PREP(KF_F32); break;
     case KF_F16: KF_PREP(KF_F16); break;

@@ -43,3 +43,21 @@ def test_planes_are_the_rounded_values(mode, hd, S, odd):
             assert torch.equal(out[1], (x.float() - hi.float()).to(st))
     assert torch.count_nonzero(vb[: 2 if two else 1, ..., S:sp]) == 0
     assert bool((kb[..., hd:] == 7).all() and (vb[..., sp:] == 7).all()), "wrote past the rows"
+
+
+@pytest.mark.parametrize("mode", [L.MMA_F16, L.MMA_F16X3])
+@pytest.mark.parametrize("hd", [8, 32, 64, 256])
+@pytest.mark.parametrize("B,H,S", [(700, 5, 4), (41, 7, 17), (300, 3, 33), (9, 3, 300)])
+def test_short_sequences_share_wavefronts(mode, hd, B, H, S):
+    """Heads of few keys packed into wavefronts, and heads that start wavefronts of their own."""
+    dt = torch.float16 if mode == L.MMA_F16 else torch.float32
+    g = torch.Generator(device=DEV).manual_seed(S)
+    k, v = (torch.randn(B, S, H, hd, device=DEV, generator=g).to(dt).permute(0, 2, 1, 3) for _ in "kv")
+    k_hi, k_lo, vt_hi, vt_lo = K.attn_prep(k, v, mode)
+    vt = v.transpose(-2, -1)
+    assert torch.equal(k_hi, k.half()) and torch.equal(vt_hi[..., :S], vt.half())
+    assert torch.count_nonzero(vt_hi[..., S:]) == 0
+    if mode == L.MMA_F16X3:
+        assert torch.equal(k_lo, (k - k.half().float()).half())
+        assert torch.equal(vt_lo[..., :S], (vt - vt.half().float()).half())
+        assert torch.count_nonzero(vt_lo[..., S:]) == 0
