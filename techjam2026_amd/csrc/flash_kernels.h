@@ -63,7 +63,8 @@ constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLazy = 8.0f;     // log2 units: probabilities stay <= 256
 
 // SMALL: one 16-row group per wavefront instead of two (64-row blocks of four wavefronts at
-// head_dim <= 32, 128-row blocks of eight at 128), for grids that leave CUs idle (launch_fwd).
+// head_dim <= 32, 128-row blocks of eight at 128), for grids that leave CUs idle (launch_fwd) and
+// for short sequences with general masks (launch_general).
 template <int HDP, int P = 2, bool SMALL = false> struct FlashTile {
   // hd 64 in the split modes: eight wavefronts of one 16-row group (the same
   // 128-row block as four of two groups) at ~100-126 VGPRs, so two blocks give each SIMD
@@ -83,7 +84,7 @@ template <int HDP, int P = 2, bool SMALL = false> struct FlashTile {
   // (C4-shape attention 0.416 -> 0.405 ms, measured on MI355X)
   static constexpr int STAGES = (HDP >= 256 && P == 1) ? 4 : (HDP >= 128 && 3 * STAGE_BYTES <= 160 * 1024) ? 3 : 2;
   static_assert(BM == (HDP == 128 ? 256 : 128) / (SMALL ? 2 : 1), "block height per head dim");
-  static_assert(!SMALL || HDP == 32 || HDP == 128, "head dims with small blocks");
+  static_assert(!SMALL || HDP == 32 || HDP == 128 || (HDP == 64 && P == 1), "tiles with small blocks");
 };
 
 __device__ __forceinline__ void store_o4(const FlashArgs& a, int64_t off, const float* v) {
@@ -830,18 +831,24 @@ void flash_fwd_kernel(FlashArgs a) {
 // packed, pipelined single pass). A few blocks a CU walk the `nblocks` of the grid, and leave
 // at once where the batch has no such row, which is the usual case: a launch of the whole
 // grid to find that out took 45 us over 32768 blocks.
-template <int MODE, int QT, int HDP, int VAR = kVarNone>
-__global__ __launch_bounds__((FlashTile<HDP, ModeTraits<MODE>::split ? 2 : 1>::NTH))
+template <int MODE, int QT, int HDP, int VAR, bool SMALL>
+__global__ __launch_bounds__((FlashTile<HDP, ModeTraits<MODE>::split ? 2 : 1, SMALL>::NTH))
 void flash_general_kernel(FlashArgs a, int nblocks) {
   __shared__ __attribute__((aligned(1024)))
   typename ModeTraits<MODE>::elem smem[flash_stage_elems<MODE, HDP>()];
   if (a.kv_len && a.prefix) {
-    int any = 0;
-    for (int b = threadIdx.x; b < a.B; b += blockDim.x) any |= a.prefix[b] == 0;
+    int any = 0;                       // eight loads in flight: one at a time, 16384 batch rows took 30 us
+    for (int b = threadIdx.x; b < a.B; b += 8 * blockDim.x) {
+      int p[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) p[i] = a.prefix[min(b + i * (int)blockDim.x, a.B - 1)];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) any |= p[i] == 0;
+    }
     if (!__syncthreads_or(any)) return;
   }
   for (int bid = blockIdx.x; bid < nblocks; bid += gridDim.x) {
-    flash_fwd_block<MODE, QT, HDP, VAR, true>(a, bid, nblocks, smem);
+    flash_fwd_block<MODE, QT, HDP, VAR, true, SMALL>(a, bid, nblocks, smem);
     lds_barrier();                     // the stages are read before the next block's copies
   }
 }
@@ -2297,16 +2304,28 @@ __global__ __launch_bounds__(SmallTile::NTH) void flash_small_kernel(FlashArgs a
 
 // The general rows of a launch whose prefix rows another kernel serves (all rows are
 // general where the extents are not given).
-template <int MODE, int QT, int HDP, int VAR = kVarNone>
-static void launch_general(FlashArgs a, hipStream_t st) {
-  if (a.keep == nullptr) return;
-  using FT = FlashTile<HDP, ModeTraits<MODE>::split ? 2 : 1>;
+template <int MODE, int QT, int HDP, int VAR, bool SMALL>
+static void launch_general_tile(FlashArgs a, hipStream_t st) {
+  using FT = FlashTile<HDP, ModeTraits<MODE>::split ? 2 : 1, SMALL>;
   const int64_t blocks = (int64_t)((a.S + FT::BM - 1) / FT::BM) * a.B * a.H;
   const int64_t resident = 4LL * cu_count();
   a.only_general = 1;
-  hipLaunchKernelGGL((flash_general_kernel<MODE, QT, HDP, VAR>),
+  hipLaunchKernelGGL((flash_general_kernel<MODE, QT, HDP, VAR, SMALL>),
                      dim3((unsigned)(blocks < resident ? blocks : resident)), dim3(FT::NTH), 0, st, a,
                      (int)blocks);
+}
+
+template <int MODE, int QT, int HDP, int VAR = kVarNone>
+static void launch_general(const FlashArgs& a, hipStream_t st) {
+  if (a.keep == nullptr) return;
+  // Sequences of up to 64 keys: 64-row blocks, one row group a wavefront. Fewer registers keep
+  // twice the blocks on a CU, whose chain of loads is the time there, and fewer wavefronts idle
+  // (left-padded, causal: 65536 heads of 4 keys of 8, f16x3, 616 -> 284 us, 4096 heads of 16 keys
+  // of 64, fp16, 46.0 -> 35.9; one block per head and launch took 464 and 38.2).
+  if constexpr (HDP == 32 || (HDP == 64 && !ModeTraits<MODE>::split)) {
+    if (a.S <= 64) return launch_general_tile<MODE, QT, HDP, VAR, true>(a, st);
+  }
+  launch_general_tile<MODE, QT, HDP, VAR, false>(a, st);
 }
 
 template <int MODE, int QT, int HDP, int VAR = kVarNone>

@@ -64,3 +64,12 @@ def test_no_mask_equals_a_mask_of_ones(mode, hd, B, H, S, causal):
     assert torch.equal(got, want)
     p16 = [K.flash_attention(q, k, v, keep=m, causal=causal, mode=mode, p16=True) for m in (None, ones)]
     assert torch.equal(*p16)
+
+
+@pytest.mark.parametrize("mode", [L.MMA_F16, L.MMA_F16X3, L.MMA_BF16X3])
+@pytest.mark.parametrize("hd", [8, 64, 128])
+@pytest.mark.parametrize("B,H,S", [(300, 5, 4), (270, 4, 33), (1030, 1, 64), (140, 8, 65)])
+def test_short_sequences_beyond_the_grid_match_float64(mode, hd, B, H, S):
+    """More (row, head) pairs than the general kernel has blocks, at and around the length up to
+    which it takes 64-row blocks."""
+    test_mixed_masks_match_float64(mode, hd, B, H, S, True)
