@@ -214,9 +214,10 @@ typedef struct {
  *   s = (s + gelu(h . W1^T + b1) . W2^T + b2) * keep
  * (without it s = res * keep); s_out, if given, receives s; h = LN(s; norm). Then with
  * KF_LAYER_QKV the projections of h in the attention layout of kf_gemm_qkv (k_lo / vt_lo
- * NULL: one plane each; the pad columns [S, sp) of v^T are zeroed), else y = h * keep in
- * y_dtype. Replaces kernelforge/optimized.py:483-489 and :560-585 for such widths, where
- * the reference launches each operation. Row results do not depend on `rows`. */
+ * NULL: one plane each; v^T's pad columns [S, roundup(S, 8)) are zeroed, those from there to sp
+ * left as they are), else y = h * keep in y_dtype. Replaces kernelforge/optimized.py:483-489
+ * and :560-585 for such widths, where the reference launches each operation. Row results do
+ * not depend on `rows`. */
 int kf_layer_block(const kf_layer_args* args, void* stream);
 
 /* k, v [B, H, S, hd] (strides[4] in elements, unit hd stride; fp32 / fp16 / bf16) into the

@@ -63,7 +63,7 @@ struct LayerArgs {
   // QKV
   const _Float16* wq_hi; const _Float16* wq_lo; const float* bq;
   float* q_out; _Float16* k_hi; _Float16* k_lo; _Float16* vt_hi; _Float16* vt_lo;
-  int64_t sp; int S, H, hd;
+  int64_t sp; int S;
   // final
   void* y; int y_dtype;
   int M, F;
@@ -556,7 +556,7 @@ void layer_kernel(LayerArgs g) {
       }
     }
     // v^T [B, d, sp]: the operands swapped, so a lane holds tokens 4 grp .. 4 grp + 3 of
-    // column r; the lane that has a sequence's last token also zeroes the pad [S, sp)
+    // column r; the lane that has a sequence's last token also zeroes the pad [S, roundup(S, 8))
     reread();
     product(acc, xa, p_qkv + 2, g.m_attn, Yes{}, Yes{});
 #pragma unroll
@@ -597,7 +597,7 @@ void layer_kernel(LayerArgs g) {
             const int64_t at = b * row + t;
             *(half4*)(vh + at) = hi;
             if (k_two) *(half4*)(vl + at) = lo;
-            if (t + 4 == g.S && g.sp > g.S) {    // S % 8 == 4: one quad of padding
+            if (t + 4 == g.S && (g.S & 4)) {     // one quad of padding to a multiple of 8
               *(half4*)(vh + at + 4) = half4{0, 0, 0, 0};
               if (k_two) *(half4*)(vl + at + 4) = half4{0, 0, 0, 0};
             }
@@ -762,7 +762,7 @@ extern "C" int kf_layer_block(const kf_layer_args* p, void* stream) {
     a.wq_lo = p->attn_mode == KF_MMA_F16 ? nullptr : (const _Float16*)p->wqkv_lo;
     a.q_out = p->q_out; a.k_hi = (_Float16*)p->k_hi; a.k_lo = (_Float16*)p->k_lo;
     a.vt_hi = (_Float16*)p->vt_hi; a.vt_lo = (_Float16*)p->vt_lo;
-    a.sp = p->sp; a.S = (int)p->S; a.H = (int)p->H; a.hd = (int)p->hd;
+    a.sp = p->sp; a.S = (int)p->S;
     uni = uni && p->attn_mode == KF_MMA_F16X3;
   } else {
     if (!p->y || p->y_dtype < KF_F32 || p->y_dtype > KF_BF16 || !al16(p->y)) {

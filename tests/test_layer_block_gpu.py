@@ -136,3 +136,22 @@ def test_single_plane_operands_are_the_rounded_values():
     two = K.layer_block(x, None, p["norm"], qkv=(w, 2, 50, 2, 32, False))[1]
     one = K.layer_block(x, None, p["norm"], qkv=(w, 2, 50, 2, 32, True))[1]
     assert one.k_lo is None and torch.equal(one.k_hi, two.k_hi) and torch.equal(one.vt_hi, two.vt_hi)
+
+
+@pytest.mark.parametrize("S", [40, 44, 45, 47])
+@pytest.mark.parametrize("d,rows", [(64, 16), (64, 32), (128, 16), (128, 64)])
+def test_wide_v_rows_keep_what_lies_past_the_pad(S, d, rows):
+    """V^T rows longer than roundup(S, 8): zeros up to there, nothing written beyond."""
+    p, rnd = _params(d, 64, 4)
+    B, s8 = 3, (S + 7) // 8 * 8
+    block = K.LayerBlock(B * S, d, DEV, None, p["norm"], want_residual=False, rows=rows,
+                         qkv=(K.PreparedLinear(*p["qkv"], L.MMA_F16X3), B, S, 2, d // 2, False))
+    x = rnd(B * S, d)
+    ops = block(x)[1]
+    wide = torch.full((2, B, 2, d // 2, s8 + 16), 7.0, dtype=torch.float16, device=DEV)
+    block.args.vt_hi, block.args.vt_lo, block.args.sp = wide[0].data_ptr(), wide[1].data_ptr(), s8 + 16
+    block(x)
+    for got, want in zip(wide, (ops.vt_hi, ops.vt_lo)):
+        assert torch.equal(got[..., :S], want[..., :S])
+        assert torch.count_nonzero(got[..., S:s8]) == 0
+        assert bool((got[..., s8:] == 7).all()), "wrote past the pad"
