@@ -36,7 +36,7 @@ def test_mixed_masks_match_float64(mode, hd, B, H, S, causal):
     dt = torch.float16 if mode == L.MMA_F16 else torch.float32
     q, k, v = (torch.randn(B, H, S, hd, device=DEV, generator=g).to(dt) for _ in range(3))
     keep = _masks(B, S, g)
-    kd = torch.randint(0, 3, (1,)).item()
+    kd = (hd + B) % 3                           # the mask as bool, fp32 or fp16
     got = K.flash_attention(q, k, v, keep=(keep, keep.float(), keep.half())[kd], causal=causal, mode=mode)
     s = torch.matmul(q.double(), k.double().transpose(-2, -1).contiguous()) * hd ** -0.5
     if causal:
