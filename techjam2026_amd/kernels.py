@@ -591,7 +591,7 @@ class LayerBlock:
                  rows: int = 0, check: bool = True):
         if check:
             _check_layer_operands(M, d, keep, norm, tail, qkv)
-        self.device = norm[0].device
+        self.shape, self.device = torch.Size((M, d)), norm[0].device
         self.s = torch.empty((M, d), dtype=torch.float32, device=device) if want_residual else None
         self.ops = None
         self.out_dtype = out_dtype
@@ -623,19 +623,21 @@ class LayerBlock:
             flops += 6.0 * M * d * d
             nbytes += M * d * (4 + 4 * (2 if ops.k_lo is not None else 1)) + 12 * d * d
         else:
+            a.y_dtype = _DT[out_dtype]
             nbytes += M * d * out_dtype.itemsize
         self.work = (f"layer_block[{M}x{d}]", flops, nbytes)
 
     def __call__(self, res: torch.Tensor):
         # a copy: another thread's call can't change the pointers between here and the launch
         a = L.LayerArgs.from_buffer_copy(self.args)
-        assert res.device == self.device and res.dtype == torch.float32 and tuple(res.shape) == (a.M, a.d) \
-            and res.stride(1) == 1
-        a.res, a.ld_res = res.data_ptr(), res.stride(0)
+        ld, unit = res.stride()
+        assert res.shape == self.shape and unit == 1 and res.dtype == torch.float32 \
+            and res.device == self.device
+        a.res, a.ld_res = res.data_ptr(), ld
         result = self.ops
         if result is None:
-            result = torch.empty((a.M, a.d), dtype=self.out_dtype, device=res.device)
-            a.y, a.y_dtype = result.data_ptr(), _DT[self.out_dtype]
+            result = torch.empty(self.shape, dtype=self.out_dtype, device=self.device)
+            a.y = result.data_ptr()
         tok = _begin(*self.work)
         st = L.lib().kf_layer_block(ctypes.byref(a), _stream())
         _end(tok)

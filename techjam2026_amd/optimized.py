@@ -533,8 +533,8 @@ def _entry_rows(rows: torch.Tensor) -> torch.Tensor:
     kernels take row strides of at least d), are not of unit stride or are not 16-byte aligned
     (16384 unaligned rows of d 1024, one layer: 1110 us a forward copied, 1165 through the unaligned
     LayerNorm path)."""
-    if (rows.stride(1) == 1 and rows.stride(0) >= rows.shape[1] and rows.stride(0) % 4 == 0
-            and rows.data_ptr() % 16 == 0):
+    ld, unit = rows.stride()
+    if unit == 1 and ld >= rows.shape[1] and ld % 4 == 0 and rows.data_ptr() % 16 == 0:
         return rows
     return rows.clone(memory_format=torch.contiguous_format)
 
