@@ -303,12 +303,14 @@ int cu_count();
 
 // erf-GELU, x * Phi(x). The lower tail Phi(-a) = erfc(a / sqrt 2) / 2 of a = |x| is one
 // exponential of a polynomial: log2 Phi(-a) is smooth, and a degree-10 minimax fit on [0, 6]
-// (weighted by Phi, so that the error of Phi itself is what is bounded) leaves 3.2e-10 in
-// Phi, far below the rounding of its fp32 evaluation. Past 6 the fit goes on falling (its
-// leading coefficient is negative), so the tail underflows to zero as it should; +-inf and
-// NaN come out as x * Phi(x) gives them. Error against float64 over N(0, 1) inputs, 2-norm:
-// 3.4e-8 relative, 0.5 x (1 + erf(x / sqrt 2)) in fp32 3.7e-8. Twelve VALU instructions and
-// one exponential with no branch, where the library erff takes both of its branches whenever a
+// (weighted by Phi, so that the error of Phi itself is what is bounded), its coefficients rounded to
+// fp32, leaves 4.8e-9 in Phi, below the rounding of its fp32 evaluation. Past 6 the fit goes on
+// falling (its leading coefficient is negative), faster than Phi does (a third below it at 8), so the
+// tail, 1e-9 and less, underflows to zero as it should; +-inf and NaN come out as x * Phi(x) gives
+// them. Error against float64, 2-norm relative, this form / 0.5 x (1 + erf(x / sqrt 2)) in fp32:
+// inputs N(0, 1) 3.4e-8 / 3.7e-8, N(0, 3^2) 2.6e-8 / 3.0e-8, N(0, 0.5^2) 4.0e-8 / 4.0e-8, and for
+// |x| < 0.1, where the exponential's last bit counts, 4.8e-8 / 3.7e-8. Fourteen VALU instructions
+// and one exponential with no branch, where the library erff takes both of its branches whenever a
 // wavefront's lanes differ (about 40 instructions).
 __device__ __forceinline__ float gelu_erf(float x) {
   const float a = __builtin_fabsf(x);

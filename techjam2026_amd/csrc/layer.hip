@@ -13,13 +13,16 @@
 // row values s stay in fp32 registers and the 16-bit operands (planes of ctx, h, the
 // hidden chunk) in LDS; only ctx and res are read and only s and the outputs written.
 //
-// What bounds it: for many rows the row arithmetic (LayerNorm, GELU, plane splits: about half
-// of the VALU's cycles at d = F = 128, the matrix cores busy a fifth), above the 12 bytes per
-// element of [M, d] it moves where separate launches move 56; for few rows the latency of the
-// chain of products. Measured on MI355X against the separate kernels: a d = F = 128 layer over
-// 10000 x 128 rows (entry block, attention, tail) 4.90 -> 2.71 ms; four such layers over one
-// 128-token sequence, replayed from a graph, 206 -> 93 us; d 64, F 256, 64 x 1024 rows
-// 190 -> 130 us; d 256, F 1024, 2 x 128 rows 76 -> 57 us (each before later changes).
+// What bounds it: for few rows the latency of the chain of products, each block streaming every
+// weight. For many rows (10000 x 128 rows of d = F = 128, f16x3; profiles/pmc_layer_kernel.txt) the
+// tail runs VALU instructions (LayerNorm, GELU, plane splits) in 52 % of the SIMDs' cycles and MFMAs
+// in 25 %, at 2.6 TB/s; the entry block 32 % and 24 %, at 3.6 TB/s, its wavefronts waiting to issue
+// for most of the rest. HBM traffic is what the operands are, each once: per element of [M, d] 16
+// bytes for an entry block, 24 for a tail with the next projections, 12 for the last tail, where
+// separate launches of that one's operations move 52. Measured on MI355X against the separate
+// kernels that it replaced: that model, one layer, 4.95 -> 2.00 ms; four layers of d = F = 128 over
+// one 128-token sequence 206 -> 69.5 us; d 64, F 256, 64 x 1024 rows 185 -> 101 us. Against today's
+// separate kernels (small GEMM tiles) see FusedTransformer.ROW_KERNEL_BYTES.
 //
 // Split: a block has d / 16 / FN wavefronts, each owning 16 FN columns of every product and all
 // BM rows. The product is formed as W . A^T, so a lane holds four

@@ -528,6 +528,8 @@ def linear_qkv(h: Act, w: PreparedLinear, B: int, S: int, H: int, Dh: int,
 
 
 # ------------------------------------------------------------------ narrow layers
+# d / 32 k-steps of a product come in whole groups of the kernel's weight ring (up to 4, then 4 or
+# 3 a group), so 160 and 224 (5 and 7 k-steps) run the separate kernels
 LAYER_WIDTHS = (32, 64, 96, 128, 192, 256)
 LAYER_MODES = (L.MMA_F16, L.MMA_F16X2, L.MMA_F16X3)
 

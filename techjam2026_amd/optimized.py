@@ -15,6 +15,9 @@ device op of the forward is a libkf950 kernel:
       gemm(f, W2)                           ffn_out
       add_mask_ln(res, ffn, keep, next)     next layer's norm1, or final_norm + mask
 
+In narrow models (`FusedTransformer._rows_fused`) one kernel, kf_layer_block, does all of a
+layer but the attention: from its output to the next layer's q, k, v^T.
+
 Precision is chosen per stage ("attn" = QKV GEMM + attention, "out_proj", "ffn1",
 "ffn2"): "f16x3" / "bf16x3" (split fp32 on the fp16/bf16 MFMA, fp32-level accuracy),
 "f16x3p" (f16x3 with the attention probabilities as one fp16 plane in P.V),
