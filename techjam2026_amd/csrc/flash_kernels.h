@@ -837,7 +837,7 @@ void flash_general_kernel(FlashArgs a, int nblocks) {
   __shared__ __attribute__((aligned(1024)))
   typename ModeTraits<MODE>::elem smem[flash_stage_elems<MODE, HDP>()];
   if (a.kv_len && a.prefix) {
-    int any = 0;                       // eight loads in flight: one at a time, 16384 batch rows took 30 us
+    int any = 0;      // eight loads in flight: 16384 batch rows of prefixes 5.6 us, one at a time 23.6
     for (int b = threadIdx.x; b < a.B; b += 8 * blockDim.x) {
       int p[8];
 #pragma unroll
