@@ -4,6 +4,8 @@ new inputs, whatever their strides and the mask's type, with eager work in betwe
 outside inference mode, one layer deep (nothing but attention is captured) and deeper."""
 from __future__ import annotations
 
+import threading
+
 import pytest
 import torch
 
@@ -78,3 +80,36 @@ def test_rows_that_overlap_or_repeat(d, H, F, layers, B, S, dtype):
                 got = graphed(form, None)
                 want = build_shared(base.config, LADDER["f16x3"], base)(dense, None)
                 assert torch.equal(got, want), what
+
+
+@pytest.mark.parametrize("d,H,F,layers", [(128, 4, 192, 1), (64, 8, 64, 2), (512, 8, 512, 2)])
+def test_threads_that_share_a_model_and_a_stream(d, H, F, layers):
+    """Each thread's calls return the forward of its own input and mask."""
+    B, S = 2, 50
+    base = make_model(TransformerConfig(B, S, d, H, F, layers, True), device=DEV)
+    eager = build_shared(base.config, LADDER["f16x3"], base)
+    graphed = build_shared(base.config, LADDER["graph"], base)
+    g = torch.Generator(device=DEV).manual_seed(5)
+    data = []
+    with torch.no_grad():
+        for _ in range(4):
+            x = torch.randn(B, S, d, device=DEV, generator=g)
+            m = torch.arange(S, device=DEV)[None] < torch.randint(1, S + 1, (B, 1), device=DEV, generator=g)
+            data.append((x, m, eager(x, m)))
+        graphed(*data[0][:2])                                # captured before the threads start
+    torch.cuda.synchronize()
+    wrong = []
+
+    def calls(i):
+        x, m, want = data[i]
+        with torch.no_grad():
+            got = [graphed(x, m) for _ in range(25)]
+        torch.cuda.synchronize()
+        wrong.extend((i, n) for n, y in enumerate(got) if not torch.equal(y, want))
+
+    threads = [threading.Thread(target=calls, args=(i,)) for i in range(len(data))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+    assert not wrong and not any(t.is_alive() for t in threads)
